@@ -76,6 +76,10 @@ extern "C" {
                                       the batch are at least the workgroups; on bf16 caches of
                                       4 KV heads, pairs of heads 0 and 3, 1 and 2 when the
                                       pairs of the batch outnumber the workgroups               */
+#define MX_SCHEDULE_TILED 4        /* blocks of 128 or 256 query rows of a KV head against K/V
+                                      tiles shared through LDS, long key ranges cut into pieces
+                                      merged in the same launch: automatic plans of many query
+                                      rows per KV head                                            */
 
 /* Phase flags for mx_paged_gqa_decode (0 = run everything). */
 #define MX_PHASE_MAIN_ONLY 1        /* split grid: run only the split-KV kernel, partials stay in

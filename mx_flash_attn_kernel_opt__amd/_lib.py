@@ -34,6 +34,7 @@ MX_SCHEDULE_SPLIT_GRID = 0
 MX_SCHEDULE_BALANCED = 1
 MX_SCHEDULE_SPLIT_GRID_PAIRED = 2
 MX_SCHEDULE_BALANCED_PAIRED = 3
+MX_SCHEDULE_TILED = 4
 
 MX_PHASE_ALL = 0
 MX_PHASE_MAIN_ONLY = 1

@@ -27,6 +27,9 @@
 //    combine kernel in a second launch only when the counters do not fit), and a
 //    length-balanced launch that cuts the batch's chunk line into equal shares on the device
 //    and merges cut units through a fan-in-8 tree of the same kind.
+//  * Many query rows per KV head (prompt chunks, long verifications, large groups) take a third
+//    kernel, tiled.h: blocks of 64 to 256 rows against K/V tiles shared through LDS, bound by
+//    the matrix cores instead of re-reading K/V for every 16 or 32 rows.
 //  * Sharded decode: the same kernels can write each query row as fp32 output plus its
 //    log-sum-exp (mx_paged_gqa_decode_partial) for a cross-device merge (mx_lse_merge).
 //  * Paged K/V append (mx_paged_kv_append), and append-and-attend (mx_paged_gqa_decode_append):
@@ -1318,7 +1321,7 @@ struct NewTokens {
 // head) does it, as its last work: the stores' completion then delays no barrier or merge of
 // the launch, and none of these slots is read unmasked by it (cache chunks cover positions
 // below SeqExtent::cache only).
-template <int D>
+template <int D, bool kFp8 = false>
 __device__ __forceinline__ void copy_new_tokens(const int32_t* __restrict__ seq_lens,
                                                 const int32_t* __restrict__ block_table, int b,
                                                 int kv, const MainShape& sh, uint32_t* status,
@@ -1348,7 +1351,13 @@ __device__ __forceinline__ void copy_new_tokens(const int32_t* __restrict__ seq_
     const int64_t dst = (int64_t)pid * sh.page_stride + (int64_t)(pos % psize) * sh.token_stride +
                         kv * D + 8 * seg;
     const u32x4 x = *reinterpret_cast<const u32x4*>((is_v ? sh.v_new : sh.k_new) + src);
-    *reinterpret_cast<u32x4*>((is_v ? sh.v_dst : sh.k_dst) + dst) = x;
+    if constexpr (kFp8) {
+      const float scale = is_v ? sh.v_scale : sh.k_scale;
+      *reinterpret_cast<u32x2*>(reinterpret_cast<uint8_t*>(is_v ? sh.v_dst : sh.k_dst) + dst) =
+          u32x2{bf16x4_to_fp8x4(x[0], x[1], scale), bf16x4_to_fp8x4(x[2], x[3], scale)};
+    } else {
+      *reinterpret_cast<u32x4*>((is_v ? sh.v_dst : sh.k_dst) + dst) = x;
+    }
   }
   if (__builtin_amdgcn_ballot_w64(overflow) != 0 && (tid & 63) == 0)
     atomicOr(status, (uint32_t)MX_DEVICE_SEQ_TOO_LONG);
@@ -1835,6 +1844,8 @@ void mx_paged_decode_splitkv(
     merge_tree<D, NW, kMergeFanIn>(tree, split, nsv, nrows, s_lse, &s_last);
   copy_if_writer();
 }
+
+#include "tiled.h"
 
 // ------------------------------------------------------------------------------------------
 // Length-balanced kernel
@@ -2369,6 +2380,32 @@ __global__ __launch_bounds__(64) void mx_paged_decode_combine(
                       pair_group > 0 ? (h / pair_group) & 1 : -1);
 }
 
+// Second launch of the tiled schedule (more than kTileFusedPieces pieces): one wave per (query head,
+// sequence * query token) merges the pieces of the row's block of block_rows rows (tile_range, with
+// the tiled launch's shape).
+template <int D>
+__global__ __launch_bounds__(256) void mx_paged_tiled_combine(
+    const float* __restrict__ part_o, const float* __restrict__ part_lse,
+    const int32_t* __restrict__ seq_lens, uint16_t* __restrict__ out, int block_rows, int kb,
+    uint32_t* __restrict__ status, const MainShape sh) {
+  const int lane = threadIdx.x & 63;
+  const int h = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+  if (h >= sh.num_heads) return;
+  const int bt = blockIdx.y;  // sequence * seqlen_q + query token
+  const int b = bt / sh.seqlen_q;
+  const int r = (bt - b * sh.seqlen_q) * sh.group + h % sh.group;
+  const int r0 = r / block_rows * block_rows;
+  const int seq = sh.new_tokens > 0 ? seq_extent<true>(seq_lens, b, sh, status, false).keys
+                                    : seq_extent<false>(seq_lens, b, sh, status, false).keys;
+  const int n = tile_range(r0, min(block_rows, sh.rows - r0), seq, kb, sh).pieces;
+  if (n == 1) return;  // the main kernel wrote it
+  const int64_t row = (int64_t)bt * sh.num_heads + h;
+  float acc[D / 64];
+  const float lse = merge_row<D>(acc, part_lse + row * sh.num_splits, 1, 1.0f,
+                                 part_o + row * sh.num_splits * D, D, n, lane);
+  store_merged_row<D>(acc, lse, out, sh.o_out, sh.lse_out, row, lane);
+}
+
 // mx_lse_merge: rows merged over `parts` gathered partials, part-major ([parts, rows, D] and
 // [parts, rows], natural-log sum-exps); one wave per row.
 template <int D>
@@ -2565,6 +2602,7 @@ struct Plan {
   int64_t slots = 0;              // balanced: partial slots (groups + units)
   int64_t rows = 1;               // query rows per KV head: seqlen_q * group
   int64_t row_tiles = 1;          // row groups: ceil(rows / (16 * tiles_per_group))
+  int tile_row_waves = 0;         // MX_SCHEDULE_TILED: row waves per workgroup (32 rows each)
   int tiles_per_group = 1;        // 16-row tiles one pass over K/V serves (1, or 2 above 16 rows)
   int64_t cap_tokens = 0;
   int64_t counter_offset = 0;
@@ -2658,7 +2696,7 @@ int64_t auto_splits(int64_t units, int64_t slots, int64_t cap) {
   return ns;
 }
 
-int make_plan(int64_t batch, int64_t seqlen_q, int64_t num_heads, int64_t num_kv_heads,
+int make_stream_plan(int64_t batch, int64_t seqlen_q, int64_t num_heads, int64_t num_kv_heads,
               int64_t head_dim, int64_t page_size, int64_t max_pages, int64_t max_seq_len,
               int64_t num_splits, int64_t num_cus, int pair_ok, Plan* plan) {
   if (batch < 1 || seqlen_q < 1 || num_heads < 1 || num_kv_heads < 1 || head_dim < 1 ||
@@ -2822,6 +2860,98 @@ int make_plan(int64_t batch, int64_t seqlen_q, int64_t num_heads, int64_t num_kv
     plan->workspace_bytes = kStatusBytes;
   }
   return MX_STATUS_OK;
+}
+
+// ---- Tiled schedule (mx_paged_attend_tiled) ----
+//
+// Automatic plans with at least this many query rows per KV head take it: more rows than one pass
+// of the streaming kernels serves (32 at head_dim 64 and 128, 16 at 256), which read a head's K/V
+// again for every further pass.  At the line, streaming against tiled (us): 33 rows, B=64, 8 KV
+// heads, 1 000-2 000 keys 137 / 94; B=4, 1 KV head 18.9 / 18.9 (the host's time); head_dim 256, 17
+// rows, B=16 26.3 / 23.3, 32 rows, B=64 at 4 096 keys 172 / 110.  Far from it: 4 prompts of 1 500
+// tokens 820 / 125, a 512-token chunk over 16K keys 518 / 167.
+constexpr int64_t tile_min_rows(int64_t head_dim) { return head_dim == 256 ? 17 : 33; }
+constexpr int64_t kTileMaxPieces = 32;      // pieces of a unit's keys
+constexpr int64_t kTileMinPieceKeys = 128;  // of capacity: two tiles
+// Up to two pieces merge in the launch (the last to arrive merges a block's rows), more in a
+// second one spread over the whole device: a 512-token chunk over 16K keys in 2 pieces of 128-row
+// blocks 175 against 186 us, in 4 pieces of 256-row blocks 175 against 163.
+constexpr int64_t kTileFusedPieces = 2;
+// Row waves per workgroup (WR).  64 rows or fewer need two.  Eight (256 rows) read K/V least often
+// and merge nothing in the workgroup, but make few, long workgroups: they win where those still
+// fill the device or the key ranges are long (4 prompts of 1 500 tokens: 116 us against 149 with
+// four and 232 with two; 1 000 tokens over 28K keys 143 / 156 / 192; a 512-token chunk over 16K
+// keys 163 / 175 / 230), and lose on the rest (1 prompt of 1 000 tokens 40 / 31 / 33; 512 tokens
+// over 2K keys 47.5 / 46.4 / 43.9; 64 tokens over 8K keys 31.6 / 29.4 / 30.4, each at its best
+// piece count).  At head_dim 256 a wave takes a SIMD's registers: four waves, two or four on rows.
+constexpr int64_t kTileLongCap = 4096;
+int tile_row_waves(int64_t batch, int64_t num_kv_heads, int64_t rows, int64_t head_dim,
+                   int64_t cap, int64_t num_cus) {
+  if (rows <= 64) return 2;
+  if (head_dim == 256 || rows <= 128) return 4;
+  const int64_t units8 = batch * num_kv_heads * ceil_div(rows, 256);
+  return units8 >= num_cus || cap >= kTileLongCap ? 8 : 4;
+}
+
+// The tiled plan over a streaming plan of the same call, whose capacity it keeps.
+void plan_tiled(int64_t batch, int64_t seqlen_q, int64_t num_heads, int64_t num_kv_heads,
+                int64_t head_dim, int64_t num_cus, Plan* plan) {
+  const int64_t cap = plan->cap_tokens;
+  const int wr = tile_row_waves(batch, num_kv_heads, plan->rows, head_dim, cap, num_cus);
+  const int64_t kb = tile_keys_of(head_dim, wr);
+  const int64_t cap_tiles = ceil_div(cap, kb);
+  plan->schedule = MX_SCHEDULE_TILED;
+  plan->tile_row_waves = wr;
+  plan->row_tiles = ceil_div(plan->rows, 32 * wr);
+  const int64_t units = batch * num_kv_heads * plan->row_tiles;
+  // Pieces per unit, for the shortest modelled time: rounds of workgroups, each streaming cap / n
+  // keys at the rate a workgroup measured (keys per us with every CU busy) after about 5 us of
+  // start and end, and the partials written and read back at 2 MB/us.  At most times n fills
+  // the device once (units * n <= CUs) or is 1.
+  const int64_t slots = num_cus * (head_dim == 64 && wr < 8 ? 2 : 1);  // resident workgroups
+  const double rate = (wr == 8 ? 33. : wr == 4 ? 52. : 68.) *
+                      (head_dim == 64 ? 2. : head_dim == 128 ? 1. : 0.35);
+  const int64_t row_bytes = batch * seqlen_q * num_heads * head_dim * 4;
+  int64_t best = 1;
+  double best_us = 0.;
+  for (int64_t n = 1; n <= kTileMaxPieces && (n == 1 || cap >= n * kTileMinPieceKeys); ++n) {
+    const double us = ceil_div(units * n, slots) * (cap / (n * rate) + 5.) +
+                      (n > 1 ? row_bytes * n * 0.5e-6 + (n > kTileFusedPieces ? 4. : 2.) : 0.);
+    if (n == 1 || us < best_us) {
+      best = n;
+      best_us = us;
+    }
+  }
+  const int64_t per_piece = ceil_div(cap_tiles, best);
+  int64_t ns = ceil_div(cap_tiles, per_piece);
+  const int64_t prow = batch * seqlen_q * num_heads * ns;
+  if (!split_tree_fits(units, ns, prow * head_dim * 4)) ns = 1;
+  plan->splits = ns;
+  plan->tokens_per_split = ns > 1 ? per_piece * kb : cap_tiles * kb;
+  plan->groups = plan->slots = 0;
+  plan->lse_offset = plan->o_offset = 0;
+  plan->workspace_bytes = kStatusBytes;
+  if (ns > 1) {
+    plan->lse_offset = kPartialBase;
+    plan->o_offset = kPartialBase + align_up(prow * 4, 256);
+    plan->workspace_bytes = plan->o_offset + prow * head_dim * 4;
+  }
+}
+
+// The plan of a call: the streaming plan, or the tiled one where the call allows it (tile_ok) and
+// has the rows for it.
+int make_plan(int64_t batch, int64_t seqlen_q, int64_t num_heads, int64_t num_kv_heads,
+              int64_t head_dim, int64_t page_size, int64_t max_pages, int64_t max_seq_len,
+              int64_t num_splits, int64_t num_cus, int pair_ok, bool tile_ok, Plan* plan) {
+  int st = make_stream_plan(batch, seqlen_q, num_heads, num_kv_heads, head_dim, page_size,
+                            max_pages, max_seq_len, num_splits, num_cus, pair_ok, plan);
+  if (st != MX_STATUS_OK || !tile_ok || num_splits != 0 ||
+      seqlen_q * (num_heads / num_kv_heads) < tile_min_rows(head_dim))
+    return st;
+  if (num_cus <= 0) st = query_num_cus(&num_cus);
+  if (st == MX_STATUS_OK)
+    plan_tiled(batch, seqlen_q, num_heads, num_kv_heads, head_dim, num_cus, plan);
+  return st;
 }
 
 // Library-owned workspace, one per device, grow-only (as submission_clean.cu:478-491).  A grown
@@ -3015,6 +3145,54 @@ hipError_t launch(const Plan& plan, const void* q, const void* k, const void* v,
   const uint8_t* k8 = static_cast<const uint8_t*>(k);
   const uint8_t* v8 = static_cast<const uint8_t*>(v);
 
+  if (plan.schedule == MX_SCHEDULE_TILED) {
+    // Rows above one pass of the streaming kernels: KT = 2, or 1 at head_dim 256 (tile_min_rows).
+    if (phase == MX_PHASE_COMBINE_ONLY) return hipSuccess;  // the main phase did everything
+    if constexpr (KT == (D == 256 ? 1 : 2)) {
+      sh.split_groups = (int)ceil_div(plan.splits, kMergeFanIn);
+      sh.fused_combine = plan.splits <= kTileFusedPieces ? 1 : 0;
+      const dim3 grid((unsigned)(kernel_kv * plan.row_tiles), (unsigned)batch,
+                      (unsigned)plan.splits);
+      auto go = [&](auto kernel, auto kc, auto vc) {
+        hipLaunchKernelGGL(kernel, grid, dim3(64 * tile_waves<D>()), 0, stream, q16, kc, vc,
+                           static_cast<uint16_t*>(out), seq_lens, block_table,
+                           reinterpret_cast<float*>(ws + plan.o_offset),
+                           reinterpret_cast<float*>(ws + plan.lse_offset),
+                           reinterpret_cast<uint32_t*>(ws + kStatusBytes + kXcdMaskBytes),
+                           status, sh);
+      };
+      auto pick = [&](auto wr) {
+        constexpr int WR = decltype(wr)::value;
+        if (kv.fp8 && append)
+          go(mx_paged_attend_tiled<D, WR, kCausal, true, true>, k8, v8);
+        else if (kv.fp8)
+          go(mx_paged_attend_tiled<D, WR, kCausal, true, false>, k8, v8);
+        else if (append)
+          go(mx_paged_attend_tiled<D, WR, kCausal, false, true>, k16, v16);
+        else
+          go(mx_paged_attend_tiled<D, WR, kCausal, false, false>, k16, v16);
+      };
+      if (plan.tile_row_waves == 2)
+        pick(std::integral_constant<int, 2>{});
+      else if (plan.tile_row_waves == 4)
+        pick(std::integral_constant<int, 4>{});
+      else if constexpr (D != 256)
+        pick(std::integral_constant<int, 8>{});
+      hipError_t e = hipGetLastError();
+      if (e == hipSuccess && plan.splits > 1 && !sh.fused_combine) {
+        const dim3 cgrid((unsigned)ceil_div(num_heads, 4), (unsigned)(batch * seqlen_q));
+        hipLaunchKernelGGL(mx_paged_tiled_combine<D>, cgrid, dim3(256), 0, stream,
+                           reinterpret_cast<const float*>(ws + plan.o_offset),
+                           reinterpret_cast<const float*>(ws + plan.lse_offset), seq_lens,
+                           static_cast<uint16_t*>(out), 32 * plan.tile_row_waves,
+                           (int)tile_keys_of(D, plan.tile_row_waves), status, sh);
+        e = hipGetLastError();
+      }
+      return e;
+    } else {
+      return hipErrorInvalidValue;
+    }
+  }
   if (plan.schedule == MX_SCHEDULE_BALANCED || plan.schedule == MX_SCHEDULE_BALANCED_PAIRED) {
     // One launch does everything; MX_PHASE_COMBINE_ONLY has nothing left to do.
     if (phase == MX_PHASE_COMBINE_ONLY) return hipSuccess;
@@ -3120,7 +3298,7 @@ hipError_t launch(const Plan& plan, const void* q, const void* k, const void* v,
 extern "C" {
 
 // The plan of a bf16 (fp8 = false) or fp8 cache call.
-static int report_plan(bool fp8, int64_t batch, int64_t seqlen_q, int64_t num_heads,
+static int report_plan(bool fp8, bool tile_ok, int64_t batch, int64_t seqlen_q, int64_t num_heads,
                        int64_t num_kv_heads, int64_t head_dim, int64_t page_size,
                        int64_t max_pages_per_seq, int64_t max_seq_len, int64_t num_splits,
                        int64_t num_cus, int64_t* schedule_out, int64_t* splits_out,
@@ -3130,7 +3308,7 @@ static int report_plan(bool fp8, int64_t batch, int64_t seqlen_q, int64_t num_he
   const KernelHeads kh = kernel_heads(seqlen_q, num_heads, num_kv_heads, head_dim, fp8);
   const int st = make_plan(batch, seqlen_q, num_heads, kh.kv_heads, kh.head_dim, page_size,
                            max_pages_per_seq, max_seq_len, num_splits, num_cus,
-                           pair_ok_for(fp8, kh), &plan);
+                           pair_ok_for(fp8, kh), tile_ok, &plan);
   if (st != MX_STATUS_OK) return st;
   if (schedule_out) *schedule_out = plan.schedule;
   if (splits_out) *splits_out = plan.splits;
@@ -3150,7 +3328,7 @@ int mx_paged_gqa_decode_plan(int64_t batch, int64_t seqlen_q, int64_t num_heads,
                              int64_t num_cus, int64_t* schedule_out, int64_t* splits_out,
                              int64_t* tokens_per_split_out, int64_t* workgroups_out,
                              int64_t* workspace_bytes_out) {
-  return report_plan(false, batch, seqlen_q, num_heads, num_kv_heads, head_dim, page_size,
+  return report_plan(false, true, batch, seqlen_q, num_heads, num_kv_heads, head_dim, page_size,
                      max_pages_per_seq, max_seq_len, num_splits, num_cus, schedule_out,
                      splits_out, tokens_per_split_out, workgroups_out, workspace_bytes_out);
 }
@@ -3161,7 +3339,7 @@ int mx_paged_gqa_decode_plan_fp8kv(int64_t batch, int64_t seqlen_q, int64_t num_
                                    int64_t num_splits, int64_t num_cus, int64_t* schedule_out,
                                    int64_t* splits_out, int64_t* tokens_per_split_out,
                                    int64_t* workgroups_out, int64_t* workspace_bytes_out) {
-  return report_plan(true, batch, seqlen_q, num_heads, num_kv_heads, head_dim, page_size,
+  return report_plan(true, true, batch, seqlen_q, num_heads, num_kv_heads, head_dim, page_size,
                      max_pages_per_seq, max_seq_len, num_splits, num_cus, schedule_out,
                      splits_out, tokens_per_split_out, workgroups_out, workspace_bytes_out);
 }
@@ -3173,13 +3351,15 @@ int64_t mx_paged_gqa_decode_workspace_size(int64_t batch, int64_t seqlen_q, int6
   // The size covers the call on a bf16 and on an fp8 cache (whose kernel heads may differ).
   int64_t bytes = 0;
   for (const bool fp8 : {false, true}) {
-    Plan plan;
-    const KernelHeads kh = kernel_heads(seqlen_q, num_heads, num_kv_heads, head_dim, fp8);
-    const int st = make_plan(batch, seqlen_q, num_heads, kh.kv_heads, kh.head_dim, page_size,
-                             max_pages_per_seq, max_seq_len, num_splits, 0, pair_ok_for(fp8, kh),
-                             &plan);
-    if (st != MX_STATUS_OK) return st;
-    bytes = std::max(bytes, plan.workspace_bytes);
+    for (const bool tile_ok : {false, true}) {
+      Plan plan;
+      const KernelHeads kh = kernel_heads(seqlen_q, num_heads, num_kv_heads, head_dim, fp8);
+      const int st = make_plan(batch, seqlen_q, num_heads, kh.kv_heads, kh.head_dim, page_size,
+                               max_pages_per_seq, max_seq_len, num_splits, 0,
+                               pair_ok_for(fp8, kh), tile_ok, &plan);
+      if (st != MX_STATUS_OK) return st;
+      bytes = std::max(bytes, plan.workspace_bytes);
+    }
   }
   ok();
   return bytes;
@@ -3195,7 +3375,7 @@ int prepare_decode(const void* q, const void* k_cache, const void* v_cache, cons
                    int64_t head_dim, int64_t page_size, int64_t num_pages,
                    int64_t max_pages_per_seq, int64_t max_seq_len, int32_t causal, float scale,
                    int64_t num_splits, void** workspace, int64_t workspace_bytes,
-                   int32_t phase, void* stream, int pair_ok, Plan* plan) {
+                   int32_t phase, void* stream, int pair_ok, bool tile_ok, Plan* plan) {
   if (phase != 0 && phase != MX_PHASE_MAIN_ONLY && phase != MX_PHASE_COMBINE_ONLY)
     return fail(MX_STATUS_INVALID_ARGUMENT, "phase must be 0, 1 or 2");
   // The kernels read q, K and V rows as 16-byte vectors and write out in 8-byte pieces.
@@ -3207,9 +3387,19 @@ int prepare_decode(const void* q, const void* k_cache, const void* v_cache, cons
   if (causal != 0 && causal != 1) return fail(MX_STATUS_INVALID_ARGUMENT, "causal must be 0 or 1");
   if (!std::isfinite(scale)) return fail(MX_STATUS_INVALID_ARGUMENT, "scale must be finite");
   if (num_pages < 0) return fail(MX_STATUS_INVALID_SHAPE, "num_pages must be >= 0");
+  // The tiled kernel masks unscaled scores with -inf, which a zero scale would turn into NaN.
+  tile_ok = tile_ok && fabsf(scale) >= 1e-30f;
   int st = make_plan(batch, seqlen_q, num_heads, num_kv_heads, head_dim, page_size,
-                     max_pages_per_seq, max_seq_len, num_splits, 0, pair_ok, plan);
+                     max_pages_per_seq, max_seq_len, num_splits, 0, pair_ok, tile_ok, plan);
   if (st != MX_STATUS_OK) return st;
+  if (*workspace != nullptr && workspace_bytes < plan->workspace_bytes &&
+      plan->schedule == MX_SCHEDULE_TILED) {
+    // A workspace that holds the other schedules' partials only.
+    *plan = Plan{};
+    st = make_plan(batch, seqlen_q, num_heads, num_kv_heads, head_dim, page_size,
+                   max_pages_per_seq, max_seq_len, num_splits, 0, pair_ok, false, plan);
+    if (st != MX_STATUS_OK) return st;
+  }
   if (*workspace != nullptr) {
     if (workspace_bytes < plan->workspace_bytes)
       return fail(MX_STATUS_WORKSPACE_TOO_SMALL,
@@ -3273,7 +3463,7 @@ int decode_impl(const void* q, const void* k_cache, const void* v_cache, void* o
                                 kh.kv_heads, kh.head_dim, page_size, num_pages, max_pages_per_seq,
                                 max_seq_len, causal, scale, num_splits, &workspace,
                                 workspace_bytes, phase, stream, pair_ok_for(kv.fp8, kh),
-                                &plan);
+                                /*tile_ok=*/true, &plan);
   if (st != MX_STATUS_OK) return st;
   return run_decode(plan, q, k_cache, v_cache, out, o_out, lse_out, seq_lens, block_table, batch,
                     seqlen_q, num_heads, kh.kv_heads, kh.head_dim, page_size, num_pages,
@@ -3431,10 +3621,11 @@ int mx_paged_gqa_decode_noalloc(const void* q, const void* k_cache, const void* 
     return fail(MX_STATUS_NULL_POINTER,
                 "q, k_cache, v_cache, out, seq_lens and block_table must be non-NULL");
   // The size check comes first, so a call that cannot run changes nothing on the device.  It
-  // sizes the bf16 plan that decode_impl runs (not mx_paged_gqa_decode_workspace_size, which
-  // also covers the fp8 plan's kernel heads and can be twice as large at head_dim 64).
+  // sizes the streaming plan of the bf16 call, which decode_impl falls back to where the tiled
+  // plan's partials do not fit (not mx_paged_gqa_decode_workspace_size, which also covers the fp8
+  // plan's kernel heads and can be twice as large at head_dim 64).
   int64_t need = 0;
-  const int pst = report_plan(false, batch, seqlen_q, num_heads, num_kv_heads, head_dim,
+  const int pst = report_plan(false, false, batch, seqlen_q, num_heads, num_kv_heads, head_dim,
                               page_size, max_pages_per_seq, max_seq_len, num_splits, 0, nullptr,
                               nullptr, nullptr, nullptr, &need);
   if (pst != MX_STATUS_OK) return pst;
@@ -3637,7 +3828,7 @@ static int decode_append_impl(const void* q, const void* k_new, const void* v_ne
   st = prepare_decode(q, k_cache, v_cache, out, batch, seqlen_q, num_heads, kh.kv_heads,
                       kh.head_dim, page_size, num_pages, max_pages_per_seq, max_seq_len, causal,
                       scale, num_splits, &workspace, workspace_bytes, 0, stream,
-                      pair_ok_for(kv.fp8, kh), &plan);
+                      pair_ok_for(kv.fp8, kh), /*tile_ok=*/true, &plan);
   if (st != MX_STATUS_OK) return st;
   AppendArgs app;
   if (seqlen_new >= 1 && seqlen_new <= kChunk) {

@@ -21,6 +21,7 @@ MERGE_FAN_IN = 8             # kMergeFanIn in csrc/paged_decode.hip
 MAX_MERGE_ITEMS = 8 ** 4     # kMaxMergeItems
 COUNTER_SLOTS = 4096 + 8192  # kMaxSlots in csrc/paged_decode.hip
 MAX_HANDOFF_BYTES = 2**31 - 1  # kMaxHandoffBytes
+TILED_FUSED_PIECES = 2       # kTileFusedPieces
 
 
 def _ptr(t: torch.Tensor | None) -> ctypes.c_void_p:
@@ -45,9 +46,9 @@ def plan(batch: int, num_heads: int, num_kv_heads: int, head_dim: int, page_size
     (e4m3fn) cache.
 
     Returns ``{"schedule", "splits", "tokens_per_split", "workgroups", "workspace_bytes",
-    "launches"}`` (schedule: "split_grid", "balanced", or either with "_paired": adjacent KV
-    heads in pairs; launches: kernels a phase-0 call runs);
-    raises MXAttnError for an invalid or unsupported shape.
+    "launches"}`` (schedule: "split_grid", "balanced", either with "_paired": adjacent KV
+    heads in pairs, or "tiled": many query rows per KV head; launches: kernels a phase-0 call
+    runs); raises MXAttnError for an invalid or unsupported shape.
     """
     lib = _lib.load()
     sch, ns, tps, wgs, ws = (ctypes.c_int64() for _ in range(5))
@@ -58,7 +59,8 @@ def plan(batch: int, num_heads: int, num_kv_heads: int, head_dim: int, page_size
     _lib.check(st)
     schedule = {_lib.MX_SCHEDULE_SPLIT_GRID: "split_grid", _lib.MX_SCHEDULE_BALANCED: "balanced",
                 _lib.MX_SCHEDULE_SPLIT_GRID_PAIRED: "split_grid_paired",
-                _lib.MX_SCHEDULE_BALANCED_PAIRED: "balanced_paired"}[sch.value]
+                _lib.MX_SCHEDULE_BALANCED_PAIRED: "balanced_paired",
+                _lib.MX_SCHEDULE_TILED: "tiled"}[sch.value]
     # Launches of a phase-0 call: the balanced schedule and the split grid with one split are
     # one launch; the split grid merges its splits through an in-kernel tree when there are at
     # most MAX_MERGE_ITEMS, every unit's ceil(splits / MERGE_FAN_IN) arrival counters fit the
@@ -71,6 +73,8 @@ def plan(batch: int, num_heads: int, num_kv_heads: int, head_dim: int, page_size
            (ns.value > MAX_MERGE_ITEMS or
             units * math.ceil(ns.value / MERGE_FAN_IN) > COUNTER_SLOTS or
             o_bytes > MAX_HANDOFF_BYTES))
+    if schedule == "tiled":  # more pieces than the launch merges: a combine kernel follows
+        two = ns.value > TILED_FUSED_PIECES
     return {"schedule": schedule, "splits": ns.value, "tokens_per_split": tps.value,
             "workgroups": wgs.value, "workspace_bytes": ws.value, "launches": 2 if two else 1}
 

@@ -1,0 +1,215 @@
+"""The tiled schedule (many query rows per KV head) against the CPU oracle.
+
+Sizes sit where the kernel can go wrong: row counts around its first block (33), its 32-row waves
+and its blocks of 64, 128 and 256 rows; key counts around a tile (32 or 64 keys) and a page; pieces
+merged in the launch and in a second one; the fused append, whose new rows start inside a tile.
+Tolerance: the package's own (max-abs <= 2e-2, mean-abs <= 2e-3 on bf16 outputs of N(0, 1) values).
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from conftest import assert_close_to_oracle
+from mx_flash_attn_kernel_opt__amd import (_lib, lse_merge, make_workspace, paged_gqa_decode,
+                                           paged_gqa_decode_append, paged_gqa_decode_partial, plan,
+                                           read_device_status, shard_pages)
+from mx_flash_attn_kernel_opt__amd import workloads as W
+from oracle import (paged_decode_append_reference, paged_decode_fp8_reference,
+                    paged_decode_reference, paged_kv_append_reference)
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+LENS = [0, 1, 31, 32, 33, 63, 64, 65, 100, 700]
+
+
+def _inputs(lens, G, Hkv, D, P, sq, seed=0, max_pages=None):
+    spec = W.custom_spec("tiled", lens, G * Hkv, Hkv, D, P, max_pages=max_pages, seqlen_q=sq)
+    return W.make_inputs(spec, seed=seed, device=DEV)
+
+
+def _plan(inp, fp8=False):
+    s = inp.spec
+    return plan(s.batch, s.num_heads, s.num_kv_heads, s.head_dim, s.page_size, s.max_pages,
+                seqlen_q=s.seqlen_q, fp8=fp8)
+
+
+def _oracle(inp, causal, k=None, v=None):
+    return paged_decode_reference(inp.q.cpu(), (inp.k_cache if k is None else k).cpu(),
+                                  (inp.v_cache if v is None else v).cpu(),
+                                  inp.block_table.cpu(), inp.seq_lens.cpu(), inp.scale,
+                                  causal=causal)
+
+
+def _run(inp, **kw):
+    return paged_gqa_decode(inp.q, inp.k_cache, inp.v_cache, inp.block_table, inp.seq_lens,
+                            inp.scale, **kw)
+
+
+@pytest.mark.parametrize("G,sq", [(33, 1), (4, 16), (5, 13), (128, 1), (3, 43), (1, 256), (7, 37),
+                                  (4, 129)])
+@pytest.mark.parametrize("D,P", [(64, 16), (128, 16), (128, 64), (256, 32)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_row_blocks_and_tile_edges(causal, D, P, G, sq):
+    inp = _inputs(LENS, G, 2, D, P, sq, seed=G + sq)
+    assert _plan(inp)["schedule"] == "tiled"
+    label = f"tiled D={D} P={P} G={G} sq={sq} causal={causal}"
+    print(label, flush=True)
+    out = _run(inp, causal=causal)
+    assert_close_to_oracle(out, _oracle(inp, causal), label)
+    if causal:
+        for b, L in enumerate(LENS):  # query tokens before the first key are exact zeros
+            dead = max(0, min(sq, sq - L))
+            assert not out.view(len(LENS), sq, -1)[b, :dead].float().abs().any().item()
+    assert torch.equal(out, _run(inp, causal=causal))
+    assert read_device_status() == 0
+
+
+@pytest.mark.parametrize("D,G,sq", [(256, 17, 1), (256, 4, 5), (128, 33, 1)])
+def test_first_rows_that_take_it(D, G, sq):
+    """The line itself, and one row below it the streaming schedules."""
+    inp = _inputs(LENS, G, 1, D, 16, sq, seed=3)
+    assert _plan(inp)["schedule"] == "tiled"
+    assert plan(len(LENS), G - 1 if sq == 1 else G, 1, D, 16, 44,
+                seqlen_q=1 if sq == 1 else 4)["schedule"] != "tiled"
+    assert_close_to_oracle(_run(inp), _oracle(inp, False), f"D={D} G={G} sq={sq}")
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("lens,G,Hkv,sq,pieces", [
+    ([9000], 4, 1, 40, (20, 32)),              # the second launch merges them
+    ([5000, 1, 0, 260] * 6, 8, 4, 17, (2, 5)),  # few pieces (two: merged in the launch)
+])
+def test_pieces(lens, G, Hkv, sq, pieces, D):
+    inp = _inputs(lens, G, Hkv, D, 16, sq, seed=D)
+    p = _plan(inp)
+    assert p["schedule"] == "tiled" and pieces[0] <= p["splits"] <= pieces[1], p
+    assert p["launches"] == (2 if p["splits"] > 2 else 1)
+    label = f"pieces D={D} {p}"
+    print(label, flush=True)
+    out = _run(inp, causal=True).clone()
+    assert_close_to_oracle(out, _oracle(inp, True), label)
+    for _ in range(3):  # whichever workgroup merges, the same bits
+        assert torch.equal(_run(inp, causal=True), out)
+    # partial outputs of two shards, merged
+    shards = shard_pages(inp.block_table, inp.seq_lens, 16, 2, sq)
+    parts = [paged_gqa_decode_partial(inp.q, inp.k_cache, inp.v_cache, t, l, inp.scale,
+                                      causal=i == 1) for i, (t, l) in enumerate(shards)]
+    merged = lse_merge(torch.stack([o for o, _ in parts]), torch.stack([s for _, s in parts]))
+    assert_close_to_oracle(merged, _oracle(inp, True), "sharded " + label)
+    assert read_device_status() == 0
+
+
+@pytest.mark.parametrize("scale", [-0.07, 0.0, 1e-33])
+def test_signs_and_zero_of_the_scale(scale):
+    inp = _inputs([1, 64, 200], 8, 2, 128, 16, 9, seed=8)
+    out = paged_gqa_decode(inp.q, inp.k_cache, inp.v_cache, inp.block_table, inp.seq_lens, scale,
+                           causal=True)
+    ref = paged_decode_reference(inp.q.cpu(), inp.k_cache.cpu(), inp.v_cache.cpu(),
+                                 inp.block_table.cpu(), inp.seq_lens.cpu(), scale, causal=True)
+    assert_close_to_oracle(out, ref, f"scale {scale}")
+
+
+def test_unused_slots_do_not_reach_the_output():
+    """NaN past the sequences' ends (the rest of their last pages, and pages of no sequence)."""
+    inp = _inputs([1, 33, 64, 70], 8, 2, 128, 64, 9, seed=9)
+    ref = _oracle(inp, True)
+    used = torch.zeros(inp.k_cache.shape[:2], dtype=torch.bool, device=DEV)
+    for b, L in enumerate(inp.seq_lens.tolist()):
+        for t in range(L):
+            used[inp.block_table[b, t // 64], t % 64] = True
+    for c in (inp.k_cache, inp.v_cache):
+        c[~used] = float("nan")
+    out = _run(inp, causal=True)
+    assert_close_to_oracle(out, ref, "NaN in unused slots")
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("D,P,G,S,sq", [(128, 16, 4, 16, 16), (128, 32, 33, 1, 1), (64, 16, 8, 9, 9),
+                                        (256, 16, 8, 5, 3), (128, 16, 4, 17, 17),
+                                        (128, 64, 2, 70, 70), (64, 256, 5, 40, 40),
+                                        (128, 16, 128, 3, 4)])
+def test_append_and_attend(D, P, G, S, sq, fp8):
+    """Up to 16 new tokens in the one launch, more after the append kernel: pools bit-exact."""
+    lens = [0, 1, 15, 48, 63, 64, 65, 500, -2]
+    Hkv, B = 2, len(lens)
+    width = (500 + S) // P + 2
+    g = torch.Generator().manual_seed(S + D)
+    mk = lambda *shape: torch.randn(*shape, generator=g).to(torch.bfloat16)  # noqa: E731
+    k, v = mk(B * width, P, Hkv, D), mk(B * width, P, Hkv, D)
+    table = torch.randperm(B * width, generator=g).to(torch.int32).view(B, width)
+    kn, vn, q = mk(B, S, Hkv, D), mk(B, S, Hkv, D), mk(B, sq, G * Hkv, D)
+    lens_t = torch.tensor(lens, dtype=torch.int32)
+    assert plan(B, G * Hkv, Hkv, D, P, width, seqlen_q=sq, fp8=fp8)["schedule"] == "tiled"
+    label = f"tiled append D={D} P={P} G={G} S={S} sq={sq} fp8={fp8}"
+    print(label, flush=True)
+    kw = {}
+    if fp8:
+        kw = dict(k_scale=0.75, v_scale=1.25)
+        k, v = k.to(torch.float8_e4m3fn), v.to(torch.float8_e4m3fn)
+        k2, v2, flags = paged_kv_append_reference(kn, vn, k, v, table, lens_t, **kw)
+        ref = paged_decode_fp8_reference(q, k2, v2, table, lens_t.clamp(min=0) + S, causal=True,
+                                         **kw)
+    else:
+        ref, k2, v2, flags = paged_decode_append_reference(q, kn, vn, k, v, table, lens_t,
+                                                           causal=True)
+    assert not flags
+    kd, vd = k.to(DEV), v.to(DEV)
+    out = paged_gqa_decode_append(q.to(DEV), kn.to(DEV), vn.to(DEV), kd, vd, table.to(DEV),
+                                  lens_t.to(DEV), causal=True, **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(kd.cpu().view(torch.uint8), k2.view(torch.uint8))
+    assert torch.equal(vd.cpu().view(torch.uint8), v2.view(torch.uint8))
+    assert_close_to_oracle(out, ref, label)
+    assert read_device_status() == 0
+
+
+def test_workspace_of_the_streaming_plan_still_serves():
+    """A workspace too small for the tiled partials but not for the streaming plan's runs the
+    latter; a too small one is refused as before."""
+    inp = _inputs([6000], 4, 1, 128, 16, 40, seed=12)
+    need = _plan(inp)["workspace_bytes"]
+    ref = _oracle(inp, True)
+    for nbytes in (need, need - 256, 1 << 20):
+        ws = make_workspace(nbytes, DEV)
+        try:
+            out = _run(inp, causal=True, workspace=ws)
+        except _lib.MXAttnError as e:
+            assert e.status == _lib.MX_STATUS_WORKSPACE_TOO_SMALL and nbytes < need
+            continue
+        assert_close_to_oracle(out, ref, f"workspace of {nbytes} of {need} bytes")
+    with pytest.raises(_lib.MXAttnError):
+        _run(inp, causal=True, workspace=make_workspace(4096, DEV))
+
+
+def test_bad_pages_and_long_lengths_are_flagged():
+    inp = _inputs([300, 130], 8, 2, 128, 16, 8, seed=13, max_pages=20)
+    bt, lens = inp.block_table.clone(), inp.seq_lens.clone()
+    bt[0, 3] = 10 ** 6
+    lens[1] = 20 * 16 + 5
+    out = paged_gqa_decode(inp.q, inp.k_cache, inp.v_cache, bt, lens, inp.scale, causal=True)
+    assert read_device_status() == _lib.MX_DEVICE_BAD_PAGE_ID | _lib.MX_DEVICE_SEQ_TOO_LONG
+    bt[0, 3] = 0                 # what the kernel reads instead
+    lens[1] = 20 * 16
+    ref = paged_decode_reference(inp.q.cpu(), inp.k_cache.cpu(), inp.v_cache.cpu(), bt.cpu(),
+                                 lens.cpu(), inp.scale, causal=True)
+    assert_close_to_oracle(out, ref, "flagged page and length")
+
+
+def test_captured_calls_replay():
+    inp = _inputs([9000, 40], 4, 1, 128, 16, 40, seed=14)
+    eager = _run(inp, causal=True).clone()
+    ws = make_workspace(_plan(inp)["workspace_bytes"], DEV)
+    out = torch.empty_like(inp.q)
+    _run(inp, causal=True, out=out, workspace=ws)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        _run(inp, causal=True, out=out, workspace=ws)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+        _run(inp, causal=True)

@@ -603,3 +603,32 @@ def _decode_fp8(**over):
 def test_fp8_decode_rejects_invalid_arguments(over, status):
     assert _decode_fp8(**over) == status
     assert _lib.load().mx_last_status() == status
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,sq,cap,rows,pieces", [
+    (4, 32, 8, 128, 1500, 1504, 256, 1),      # fills the device with 256-row blocks
+    (1, 32, 8, 128, 512, 16896, 256, 4),      # long keys: 256-row blocks cut into pieces
+    (1, 32, 8, 128, 128, 2128, 128, 6),       # few rows, short keys: 128-row blocks
+    (64, 64, 1, 128, 1, 8000, 64, 4),         # 64 rows
+    (2, 16, 2, 256, 1000, 4000, 128, 1),      # head_dim 256: at most 128 rows
+])
+def test_tiled_plan_block_rows_and_pieces(B, Hq, Hkv, D, sq, cap, rows, pieces):
+    """Row blocks of 64, 128 or 256 rows, pieces that fill 256 CUs about once."""
+    p = plan(B, Hq, Hkv, D, 16, -(-cap // 16), num_cus=256, seqlen_q=sq)
+    assert p["schedule"] == "tiled" and p["splits"] == pieces, p
+    assert p["workgroups"] == B * Hkv * -(-sq * (Hq // Hkv) // rows) * pieces
+    assert p["tokens_per_split"] * pieces >= cap
+    if pieces > 1:
+        assert p["workspace_bytes"] >= B * sq * Hq * pieces * (D + 1) * 4
+    assert p["launches"] == (2 if pieces > 2 else 1)
+
+
+@pytest.mark.parametrize("D,first", [(64, 33), (128, 33), (256, 17)])
+def test_tiled_plan_starts_above_one_streaming_pass(D, first):
+    """Rows that one pass of a streaming kernel serves stay on it, and so do explicit split and
+    workgroup counts of any row count; the capacity is the streaming plan's either way."""
+    for G in (1, first - 1, first, 128):
+        p = plan(4, G, 1, D, 16, 64, num_cus=256)
+        assert (p["schedule"] == "tiled") == (G >= first)
+        assert plan(4, G, 1, D, 16, 64, 0, 2, num_cus=256)["schedule"] == "split_grid"
+        assert plan(4, G, 1, D, 16, 64, 0, -2, num_cus=256)["schedule"] == "balanced"
