@@ -39,6 +39,33 @@ def _stream_handle(stream, device: torch.device) -> ctypes.c_void_p:
     return ctypes.c_void_p(stream.cuda_stream)
 
 
+def _launch(fn, args, stream, dev: torch.device) -> None:
+    """Calls a C entry with its arguments (pointers as integers) and the stream, on ``dev``.
+
+    A small call is bound by what the host does around it, so this avoids objects: the current
+    stream's raw handle instead of a Stream (0.06 against 1.8 us), the device guard only where
+    another device is current (1.2 us).  With integer pointers, one test of a call's operands
+    and no handle objects, paged_gqa_decode went from 14.4 to 8.0 us of host time.
+    """
+    index = dev.index
+    raw = torch._C._cuda_getCurrentRawStream(index) if stream is None else stream.cuda_stream
+    if torch._C._cuda_getDevice() == index:
+        st = fn(*args, raw)
+    else:
+        with torch.cuda.device(dev):
+            st = fn(*args, raw)
+    if st != _lib.MX_STATUS_OK:
+        _lib.check(st)
+
+
+def _ready(index: int, *operands) -> bool:
+    """Whether every (tensor, dtype) operand is a contiguous tensor of that type on GPU ``index``."""
+    for t, dt in operands:
+        if t.dtype is not dt or t.get_device() != index or not t.is_contiguous():
+            return False
+    return True
+
+
 def plan(batch: int, num_heads: int, num_kv_heads: int, head_dim: int, page_size: int,
          max_pages_per_seq: int, max_seq_len: int = 0, num_splits: int = 0,
          num_cus: int = 0, seqlen_q: int = 1, fp8: bool = False) -> dict:
@@ -111,13 +138,15 @@ def _check_decode_inputs(q, k_cache, v_cache, block_table, seq_lens, allow_fp8=F
     kv_dt = torch.bfloat16
     if allow_fp8 and k_cache.dtype == torch.float8_e4m3fn:
         kv_dt = torch.float8_e4m3fn
-    for name, t, dt in (("q", q, torch.bfloat16), ("k_cache", k_cache, kv_dt),
-                        ("v_cache", v_cache, kv_dt),
-                        ("block_table", block_table, torch.int32),
-                        ("seq_lens", seq_lens, torch.int32)):
-        _require(t.device == dev, f"{name} must be on {dev}")
-        _require(t.dtype == dt, f"{name} must be {dt}, got {t.dtype}")
-        _require(t.is_contiguous(), f"{name} must be contiguous")
+    if not _ready(q.get_device(), (q, torch.bfloat16), (k_cache, kv_dt), (v_cache, kv_dt),
+                  (block_table, torch.int32), (seq_lens, torch.int32)):
+        for name, t, dt in (("q", q, torch.bfloat16), ("k_cache", k_cache, kv_dt),
+                            ("v_cache", v_cache, kv_dt),
+                            ("block_table", block_table, torch.int32),
+                            ("seq_lens", seq_lens, torch.int32)):
+            _require(t.device == dev, f"{name} must be on {dev}")
+            _require(t.dtype == dt, f"{name} must be {dt}, got {t.dtype}")
+            _require(t.is_contiguous(), f"{name} must be contiguous")
     B, SQ, Hq, D = _query_shape(q)
     _require(k_cache.dim() == 4 and k_cache.shape == v_cache.shape,
              "k_cache and v_cache must both be [num_pages, page_size, Hkv, D]")
@@ -165,22 +194,14 @@ def paged_gqa_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                  and out.device == dev, "out must be a contiguous bf16 tensor shaped like q")
     if scale is None:
         scale = 1.0 / math.sqrt(D)
-    ws_bytes = _workspace_bytes(workspace, dev)
     lib = _lib.load()
-    with torch.cuda.device(dev):
-        if fp8:
-            st = lib.mx_paged_gqa_decode_fp8kv(
-                _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(seq_lens),
-                _ptr(block_table), B, SQ, Hq, Hkv, D, P, num_pages, block_table.shape[1],
-                max_seq_len, int(bool(causal)), float(scale), float(k_scale), float(v_scale),
-                num_splits, _ptr(workspace), ws_bytes, phase, _stream_handle(stream, dev))
-        else:
-            st = lib.mx_paged_gqa_decode(
-                _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(seq_lens),
-                _ptr(block_table), B, SQ, Hq, Hkv, D, P, num_pages, block_table.shape[1],
-                max_seq_len, int(bool(causal)), float(scale), num_splits, _ptr(workspace),
-                ws_bytes, phase, _stream_handle(stream, dev))
-    _lib.check(st)
+    scales = (float(k_scale), float(v_scale)) if fp8 else ()
+    _launch(lib.mx_paged_gqa_decode_fp8kv if fp8 else lib.mx_paged_gqa_decode,
+            (q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(),
+             seq_lens.data_ptr(), block_table.data_ptr(), B, SQ, Hq, Hkv, D, P, num_pages,
+             block_table.shape[1], max_seq_len, int(bool(causal)), float(scale), *scales,
+             num_splits, 0 if workspace is None else workspace.data_ptr(),
+             _workspace_bytes(workspace, dev), phase), stream, dev)
     return out
 
 
@@ -205,14 +226,12 @@ def paged_gqa_decode_partial(q: torch.Tensor, k_cache: torch.Tensor, v_cache: to
     lse = torch.empty(q.shape[:-1], dtype=torch.float32, device=dev)
     if scale is None:
         scale = 1.0 / math.sqrt(D)
-    ws_bytes = _workspace_bytes(workspace, dev)
-    with torch.cuda.device(dev):
-        st = _lib.load().mx_paged_gqa_decode_partial(
-            _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(o), _ptr(lse), _ptr(seq_lens),
-            _ptr(block_table), B, SQ, Hq, Hkv, D, P, num_pages, block_table.shape[1],
-            max_seq_len, int(bool(causal)), float(scale), num_splits, _ptr(workspace), ws_bytes,
-            _stream_handle(stream, dev))
-    _lib.check(st)
+    _launch(_lib.load().mx_paged_gqa_decode_partial,
+            (q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), o.data_ptr(), lse.data_ptr(),
+             seq_lens.data_ptr(), block_table.data_ptr(), B, SQ, Hq, Hkv, D, P, num_pages,
+             block_table.shape[1], max_seq_len, int(bool(causal)), float(scale), num_splits,
+             0 if workspace is None else workspace.data_ptr(),
+             _workspace_bytes(workspace, dev)), stream, dev)
     return o, lse
 
 
@@ -227,14 +246,15 @@ def lse_merge(o_parts: torch.Tensor, lse_parts: torch.Tensor, *,
     """
     _require(o_parts.is_cuda, "o_parts must be a device tensor")
     dev = o_parts.device
-    for name, t in (("o_parts", o_parts), ("lse_parts", lse_parts)):
-        _require(t.device == dev, f"{name} must be on {dev}")
-        _require(t.dtype == torch.float32, f"{name} must be float32, got {t.dtype}")
-        _require(t.is_contiguous(), f"{name} must be contiguous")
-    _require(o_parts.dim() >= 2 and tuple(lse_parts.shape) == tuple(o_parts.shape[:-1]),
+    if not _ready(o_parts.get_device(), (o_parts, torch.float32), (lse_parts, torch.float32)):
+        for name, t in (("o_parts", o_parts), ("lse_parts", lse_parts)):
+            _require(t.device == dev, f"{name} must be on {dev}")
+            _require(t.dtype == torch.float32, f"{name} must be float32, got {t.dtype}")
+            _require(t.is_contiguous(), f"{name} must be contiguous")
+    _require(o_parts.dim() >= 2 and lse_parts.shape == o_parts.shape[:-1],
              "o_parts must be [parts, ..., D] and lse_parts [parts, ...]")
     parts, D = o_parts.shape[0], o_parts.shape[-1]
-    rows = o_parts[0].numel() // D if parts > 0 else 0
+    rows = lse_parts.numel() // parts if parts > 0 else 0
     shape = tuple(o_parts.shape[1:])
     if out is None:
         out = torch.empty(shape, dtype=torch.bfloat16, device=dev)
@@ -242,10 +262,8 @@ def lse_merge(o_parts: torch.Tensor, lse_parts: torch.Tensor, *,
         _require(tuple(out.shape) == shape and out.dtype == torch.bfloat16 and
                  out.is_contiguous() and out.device == dev,
                  "out must be a contiguous bf16 tensor shaped like o_parts[0]")
-    with torch.cuda.device(dev):
-        st = _lib.load().mx_lse_merge(_ptr(o_parts), _ptr(lse_parts), parts, rows, D, _ptr(out),
-                                      _stream_handle(stream, dev))
-    _lib.check(st)
+    _launch(_lib.load().mx_lse_merge, (o_parts.data_ptr(), lse_parts.data_ptr(), parts, rows, D,
+                                       out.data_ptr()), stream, dev)
     return out
 
 
@@ -329,13 +347,16 @@ def paged_kv_append(k_new: torch.Tensor, v_new: torch.Tensor, k_cache: torch.Ten
     _require(fp8 or (k_scale == 1.0 and v_scale == 1.0),
              "k_scale / v_scale apply to float8_e4m3fn caches only")
     kv_dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
-    for name, t, dt in (("k_new", k_new, torch.bfloat16), ("v_new", v_new, torch.bfloat16),
-                        ("k_cache", k_cache, kv_dt), ("v_cache", v_cache, kv_dt),
-                        ("block_table", block_table, torch.int32),
-                        ("seq_lens", seq_lens, torch.int32)):
-        _require(t.device == dev, f"{name} must be on {dev}")
-        _require(t.dtype == dt, f"{name} must be {dt}, got {t.dtype}")
-        _require(t.is_contiguous(), f"{name} must be contiguous")
+    if not _ready(k_new.get_device(), (k_new, torch.bfloat16), (v_new, torch.bfloat16),
+                  (k_cache, kv_dt), (v_cache, kv_dt), (block_table, torch.int32),
+                  (seq_lens, torch.int32)):
+        for name, t, dt in (("k_new", k_new, torch.bfloat16), ("v_new", v_new, torch.bfloat16),
+                            ("k_cache", k_cache, kv_dt), ("v_cache", v_cache, kv_dt),
+                            ("block_table", block_table, torch.int32),
+                            ("seq_lens", seq_lens, torch.int32)):
+            _require(t.device == dev, f"{name} must be on {dev}")
+            _require(t.dtype == dt, f"{name} must be {dt}, got {t.dtype}")
+            _require(t.is_contiguous(), f"{name} must be contiguous")
     _require(k_new.shape == v_new.shape, "k_new and v_new must have the same shape")
     _require(k_cache.dim() == 4 and k_cache.shape == v_cache.shape,
              "k_cache and v_cache must both be [num_pages, page_size, Hkv, D]")
@@ -354,15 +375,11 @@ def paged_kv_append(k_new: torch.Tensor, v_new: torch.Tensor, k_cache: torch.Ten
     if ws is not None:
         _require(ws.is_cuda and ws.device == dev, "workspace must be on the same device")
     lib = _lib.load()
-    common = [_ptr(k_new), _ptr(v_new), _ptr(k_cache), _ptr(v_cache), _ptr(seq_lens),
-              _ptr(block_table), B, S, Hkv, D, P, num_pages, block_table.shape[1]]
-    with torch.cuda.device(dev):
-        if fp8:
-            st = lib.mx_paged_kv_append_fp8kv(*common, float(k_scale), float(v_scale), _ptr(ws),
-                                              _stream_handle(stream, dev))
-        else:
-            st = lib.mx_paged_kv_append(*common, _ptr(ws), _stream_handle(stream, dev))
-    _lib.check(st)
+    scales = (float(k_scale), float(v_scale)) if fp8 else ()
+    _launch(lib.mx_paged_kv_append_fp8kv if fp8 else lib.mx_paged_kv_append,
+            (k_new.data_ptr(), v_new.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+             seq_lens.data_ptr(), block_table.data_ptr(), B, S, Hkv, D, P, num_pages,
+             block_table.shape[1], *scales, 0 if ws is None else ws.data_ptr()), stream, dev)
 
 
 def paged_gqa_decode_append(q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor,
@@ -388,12 +405,9 @@ def paged_gqa_decode_append(q: torch.Tensor, k_new: torch.Tensor, v_new: torch.T
     args, out, fp8 = _append_call_args(q, k_new, v_new, k_cache, v_cache, block_table,
                                        seq_lens, scale, out, causal, num_splits, max_seq_len,
                                        workspace, k_scale, v_scale)
-    dev = q.device
     lib = _lib.load()
-    fn = lib.mx_paged_gqa_decode_append_fp8kv if fp8 else lib.mx_paged_gqa_decode_append
-    with torch.cuda.device(dev):
-        st = fn(*args, _stream_handle(stream, dev))
-    _lib.check(st)
+    _launch(lib.mx_paged_gqa_decode_append_fp8kv if fp8 else lib.mx_paged_gqa_decode_append,
+            args, stream, q.device)
     return out
 
 
@@ -409,9 +423,10 @@ def _append_call_args(q, k_new, v_new, k_cache, v_cache, block_table, seq_lens, 
     _require(fp8 or (k_scale == 1.0 and v_scale == 1.0),
              "k_scale / v_scale apply to float8_e4m3fn caches only")
     _require(k_new.shape == v_new.shape, "k_new and v_new must have the same shape")
-    for name, t in (("k_new", k_new), ("v_new", v_new)):
-        _require(t.device == dev and t.dtype == torch.bfloat16 and t.is_contiguous(),
-                 f"{name} must be a contiguous bf16 tensor on {dev}")
+    if not _ready(q.get_device(), (k_new, torch.bfloat16), (v_new, torch.bfloat16)):
+        for name, t in (("k_new", k_new), ("v_new", v_new)):
+            _require(t.device == dev and t.dtype == torch.bfloat16 and t.is_contiguous(),
+                     f"{name} must be a contiguous bf16 tensor on {dev}")
     if k_new.dim() == 3:
         S = 1
         _require(tuple(k_new.shape) == (B, Hkv, D), "k_new must be [B, Hkv, D] or [B, S, Hkv, D]")
@@ -428,10 +443,11 @@ def _append_call_args(q, k_new, v_new, k_cache, v_cache, block_table, seq_lens, 
         scale = 1.0 / math.sqrt(D)
     ws_bytes = _workspace_bytes(workspace, dev)
     scales = [float(k_scale), float(v_scale)] if fp8 else []
-    args = [_ptr(q), _ptr(k_new), _ptr(v_new), _ptr(k_cache), _ptr(v_cache), _ptr(out),
-            _ptr(seq_lens), _ptr(block_table), B, SQ, S, Hq, Hkv, D, P, num_pages,
-            block_table.shape[1], max_seq_len, int(bool(causal)), float(scale), *scales,
-            num_splits, _ptr(workspace), ws_bytes]
+    args = [q.data_ptr(), k_new.data_ptr(), v_new.data_ptr(), k_cache.data_ptr(),
+            v_cache.data_ptr(), out.data_ptr(), seq_lens.data_ptr(), block_table.data_ptr(), B,
+            SQ, S, Hq, Hkv, D, P, num_pages, block_table.shape[1], max_seq_len,
+            int(bool(causal)), float(scale), *scales, num_splits,
+            0 if workspace is None else workspace.data_ptr(), ws_bytes]
     return args, out, fp8
 
 
