@@ -12,6 +12,9 @@ constexpr int tile_waves() {
 }
 constexpr int tile_keys_of(int64_t head_dim, int wr) { return head_dim == 256 || wr == 2 ? 32 : 64; }
 
+// Largest batch ordered by length (MainShape::longest_first).
+constexpr int kTileSortBatch = 512;
+
 // One 16-byte LDS segment of a tile row from the 8 elements a lane loaded.
 __device__ __forceinline__ u32x4 tile_segment(u32x4 x) { return x; }
 __device__ __forceinline__ u32x4 tile_segment(u32x2 x) {
@@ -79,6 +82,8 @@ __device__ __forceinline__ TileRange tile_range(int r0, int nrows, int seq, int 
 //    sequence's end are stored to LDS as zero V.  A wave skips tiles past its rows' last key.
 //  * One code path for masked and full tiles: instantiated twice, the compiler hoisted both tiles'
 //    operands and spilled (head_dim 128: 276 bytes per lane, 2.3 times slower).
+
+
 template <int D, int WR, bool kCausal, bool kFp8, bool kAppend>
 __global__ __launch_bounds__(64 * tile_waves<D>())
 __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2)))
@@ -115,7 +120,32 @@ void mx_paged_attend_tiled(
   // first: under a causal mask they have the most keys.
   const int kv = blockIdx.x % sh.num_kv_heads;
   const int blk = sh.row_tiles - 1 - (int)blockIdx.x / sh.num_kv_heads;
-  const int b = blockIdx.y;
+  int b = blockIdx.y;
+  // (Compiled into the 64-row blocks only: in the wider ones the code, even switched off, cost
+  // prompts 1 % and head_dim 256 chunks 4 %.)
+  if constexpr (WR == 2) {
+    if (sh.longest_first) {
+      // Workgroups start in grid order: grid row y takes the y-th longest sequence (ties by index),
+      // so the last ones to start are the shortest.  Every workgroup ranks the whole batch.
+      int* s_len = reinterpret_cast<int*>(lds);
+      for (int i = tid; i < kTileSortBatch; i += 64 * NW)
+        s_len[i] = i < sh.batch ? key_count(seq_lens, i, sh.appended) : INT_MIN;
+      __syncthreads();
+      for (int i = tid; i < sh.batch; i += 64 * NW) {
+        const int mine = s_len[i];
+        int before = 0;
+        for (int j = 0; j < sh.batch; j += 4)
+  #pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int other = s_len[j + e];
+            before += other > mine || (other == mine && j + e < i);
+          }
+        if (before == (int)blockIdx.y) s_last = i;
+      }
+      __syncthreads();
+      b = __builtin_amdgcn_readfirstlane(s_last);
+    }
+  }
   const int r0 = blk * RB;
   const int nrows = min(RB, sh.rows - r0);
 

@@ -213,3 +213,23 @@ def test_captured_calls_replay():
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
         _run(inp, causal=True)
+
+
+@pytest.mark.parametrize("G,D,fp8", [(33, 128, False), (64, 64, True), (17, 256, False)])
+def test_longest_sequences_first(G, D, fp8):
+    """More units than compute units, one row block each: grid rows follow the lengths (equal,
+    empty and negative ones among them), the outputs the sequences."""
+    lens = [(37 * i * i + 11 * i) % 300 for i in range(70)]
+    lens[3], lens[40], lens[41], lens[69] = 0, 299, 299, -4
+    inp = _inputs([max(x, 0) for x in lens], G, 8, D, 16, 1, seed=G, max_pages=19)
+    inp.seq_lens.copy_(torch.tensor(lens, dtype=torch.int32))
+    assert _plan(inp, fp8)["schedule"] == "tiled" and _plan(inp, fp8)["workgroups"] >= 560
+    if fp8:
+        k8, v8 = (c.to(torch.float8_e4m3fn) for c in (inp.k_cache, inp.v_cache))
+        out = paged_gqa_decode(inp.q, k8, v8, inp.block_table, inp.seq_lens, inp.scale)
+        ref = paged_decode_fp8_reference(inp.q.cpu(), k8.cpu(), v8.cpu(), inp.block_table.cpu(),
+                                         inp.seq_lens.cpu(), inp.scale)
+    else:
+        out, ref = _run(inp), _oracle(inp, False)
+    assert_close_to_oracle(out, ref, f"longest first G={G} D={D}")
+    assert read_device_status() == 0
