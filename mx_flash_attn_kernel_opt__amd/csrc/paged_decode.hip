@@ -2585,7 +2585,38 @@ constexpr int kMirroredPairOverhead = 10 * kChunkPositions;
 //   256 (B=128) 32.9 / 29.6 / 28.7 / 28.4 / 29.9 / 30.7.
 constexpr int kFp8UnitOverhead = 20 * kChunkPositions;
 constexpr int kFp8NarrowPairOverhead = 24 * kChunkPositions;
-constexpr int kMaxUnitOverhead = kFp8NarrowPairOverhead;  // of every charge above
+// Two row tiles (17 to 32 rows) and the new tokens of a fused append make a unit cost more chunk
+// times: a second set of queries and merged rows, and one more chunk that on fp8 caches is loaded,
+// quantized and processed after the ring.  Interleaved A/B on log-uniform lengths up to 4 000, 10 %
+// of 1-15 (B=100-256), charge taken against 64 (bf16) or 160-192 (fp8) positions, us:
+// - bf16 fused append 96: one token, 8 KV heads in pairs 58.4 -> 49.8, 2 heads 34.4 -> 30.4,
+//   head_dim 64 29.7 -> 27.6; 3 tokens 70.9 -> 60.5; mirrored pairs 128 against 80: 57.8 -> 50.6.  At
+//   head_dim 256 64 stays (96 and 160: +1, +5 %).
+// - bf16 two tiles 128: 5 query tokens 75.5 -> 63.8, groups of 24 37.6 -> 33.2; with a fused append
+//   160: 97.6 -> 68.5 (8 heads), 82.4 -> 58.9 (4), head_dim 64 29.3 -> 26.5.
+// - fp8 fused append 384: one token 54.7 -> 41.6 (8 heads), 52.2 -> 42.0 (4), 35.4 -> 29.4 (2),
+//   head_dim 64 heads in pairs 38.8 -> 31.2; head_dim 256 224: 34.8 -> 33.
+// - fp8 two tiles 224: 53.0 -> 50.5; with a fused append 448: 87.7 -> 68.2, uniform 1 000-4 000
+//   tokens 94.3 -> 84.6; head_dim 64 192: 30.8 -> 30.6.
+// Decodes of up to 16 rows without an append keep the charges above (96 against 64: 8 heads 48.0 /
+// 47.9, head_dim 64 27.1 / 27.9; fp8 256 against 160: 32.4 / 31.6).
+int unit_charge(int head_dim, int tiles, bool fp8, bool append, bool mirrored, bool narrow_pair) {
+  if (!fp8) {
+    if (tiles == 2) return (append ? 20 : 16) * kChunkPositions;
+    if (append && head_dim <= 128) return (mirrored ? 16 : 12) * kChunkPositions;
+    return mirrored ? kMirroredPairOverhead : kUnitOverhead;
+  }
+  if (append) {
+    if (head_dim == 64) return 24 * kChunkPositions;
+    if (head_dim == 256) return 28 * kChunkPositions;
+    return (tiles == 2 ? 56 : 48) * kChunkPositions;
+  }
+  if (tiles == 2) return (head_dim == 64 ? 20 : 28) * kChunkPositions;
+  return narrow_pair ? kFp8NarrowPairOverhead : kFp8UnitOverhead;
+}
+// Charge in the bound on the line's length (kBalancedMaxLine).  Larger charges stay far below 2^31
+// positions: at most kBalancedMaxUnits units.
+constexpr int kLineUnitCharge = kFp8NarrowPairOverhead;
 static_assert((kChunkPositions & (kChunkPositions - 1)) == 0,
               "the balanced kernels divide by the chunk weight with a shift");
 // Balanced schedule limits: the largest batch whose seq_lens scan stays within two passes of
@@ -2768,7 +2799,7 @@ int make_stream_plan(int64_t batch, int64_t seqlen_q, int64_t num_heads, int64_t
   plan->chunk_shift = shift;
   const int64_t units = batch * num_kv_heads * row_tiles;
   const bool balanced_ok = batch <= kBalancedMaxBatch && units <= kBalancedMaxUnits &&
-                           units * (ceil_div(cap, kChunk) * kChunkPositions + kMaxUnitOverhead) <
+                           units * (ceil_div(cap, kChunk) * kChunkPositions + kLineUnitCharge) <
                                kBalancedMaxLine;
   // Short capacities favour one split per unit (no length scan, no merge): the balanced
   // schedule pays off from 2 048 tokens, or from 1 024 with at least 512 units.
@@ -3130,9 +3161,8 @@ hipError_t launch(const Plan& plan, const void* q, const void* k, const void* v,
   sh.num_groups = (int)plan.groups;
   // A paired unit's chunk holds two heads' rows: twice a single head's weight on the line.
   sh.chunk_weight = paired ? 2 * kChunkPositions : kChunkPositions;
-  sh.unit_overhead = !kv.fp8          ? (plan.pair_mirror ? kMirroredPairOverhead : kUnitOverhead)
-                     : paired && num_kv_heads * D < 1024 ? kFp8NarrowPairOverhead
-                                                         : kFp8UnitOverhead;
+  sh.unit_overhead = unit_charge(D, KT, kv.fp8, app.new_tokens > 0, plan.pair_mirror,
+                                 paired && num_kv_heads * D < 1024);
   sh.pair_mirror = plan.pair_mirror ? 1 : 0;
   sh.num_slots = (int)plan.slots;
   sh.o_out = o_out;

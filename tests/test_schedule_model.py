@@ -157,8 +157,9 @@ def balanced_launch(lens, ups, groups, chunk_weight=8, unit_overhead=64, seed=0,
     return covered, finals, slots_of
 
 
-def _check_balanced(lens, ups, groups, chunk_weight=8, seed=0):
-    covered, finals, slots_of = balanced_launch(lens, ups, groups, chunk_weight, seed=seed)
+def _check_balanced(lens, ups, groups, chunk_weight=8, unit_overhead=64, seed=0):
+    covered, finals, slots_of = balanced_launch(lens, ups, groups, chunk_weight, unit_overhead,
+                                                seed=seed)
     _check_units(lens, ups, covered, finals, slots_of)
     return finals
 
@@ -208,6 +209,17 @@ def test_balanced_schedule_on_random_batches(seed):
 ])
 def test_balanced_schedule_on_uniform_batches(B, ups, groups, L):
     _check_balanced([L] * B, ups, groups, chunk_weight=16 if ups == 4 else 8)
+
+
+@pytest.mark.parametrize("charge", [80, 96, 128, 160, 192, 224, 384, 448])
+def test_balanced_schedule_with_every_unit_charge(charge):
+    """Charges above a unit's own chunks: whole shares may fall into one, and hold no chunk."""
+    r = random.Random(charge)
+    for seed in range(6):
+        lens = [r.choice([0, 1, 16, 17, int(math.exp(r.uniform(0, math.log(4000))))])
+                for _ in range(r.choice([3, 40, 130]))]
+        _check_balanced(lens, r.choice([1, 4, 8]), r.choice([7, 256, 512]),
+                        chunk_weight=r.choice([8, 16]), unit_overhead=charge, seed=seed)
 
 
 def test_ragged_config_shape():
