@@ -2382,16 +2382,23 @@ __global__ __launch_bounds__(64) void mx_paged_decode_combine(
                       pair_group > 0 ? (h / pair_group) & 1 : -1);
 }
 
-// Second launch of the tiled schedule (more than kTileFusedPieces pieces): one wave per (query head,
-// sequence * query token) merges the pieces of the row's block of block_rows rows (tile_range, with
-// the tiled launch's shape).
+// Second launch of the tiled schedule (more than kTileFusedPieces pieces): one wave per row merges
+// the pieces of the row's block of block_rows rows (tile_range, with the tiled launch's shape).  A
+// row's D/4 16-byte pieces leave 64 / (D/4) lane groups, which take alternate partials, four at a
+// time (loads past the last re-read it and weigh nothing), and merge their sums by lane exchanges.
+// Bound by reading the partials once.  Against one wave per row with 8-byte loads in rounds of 16
+// partials, whole calls: 16 384 rows in 4 pieces (34 MB) 159.8 -> 155.5 us, 4 096 rows in 6 pieces
+// 24.8 -> 23.5.
 template <int D>
 __global__ __launch_bounds__(256) void mx_paged_tiled_combine(
     const float* __restrict__ part_o, const float* __restrict__ part_lse,
     const int32_t* __restrict__ seq_lens, uint16_t* __restrict__ out, int block_rows, int kb,
     uint32_t* __restrict__ status, const MainShape sh) {
+  constexpr int kLanes = D / 4;        // lanes of a lane group
+  constexpr int kGroups = 64 / kLanes;
+  constexpr int W = 4;                 // partials per lane group and round
   const int lane = threadIdx.x & 63;
-  const int h = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+  const int h = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   if (h >= sh.num_heads) return;
   const int bt = blockIdx.y;  // sequence * seqlen_q + query token
   const int b = bt / sh.seqlen_q;
@@ -2402,10 +2409,54 @@ __global__ __launch_bounds__(256) void mx_paged_tiled_combine(
   const int n = tile_range(r0, min(block_rows, sh.rows - r0), seq, kb, sh).pieces;
   if (n == 1) return;  // the main kernel wrote it
   const int64_t row = (int64_t)bt * sh.num_heads + h;
-  float acc[D / 64];
-  const float lse = merge_row<D>(acc, part_lse + row * sh.num_splits, 1, 1.0f,
-                                 part_o + row * sh.num_splits * D, D, n, lane);
-  store_merged_row<D>(acc, lse, out, sh.o_out, sh.lse_out, row, lane);
+  const int d = 4 * (lane % kLanes);
+  const float* o = part_o + row * sh.num_splits * D + d;
+  const float* lse = part_lse + row * sh.num_splits;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  float wsum = 0.f, mx = -INFINITY;
+  for (int at = lane / kLanes; at < n; at += W * kGroups) {
+    float ls[W];
+    f32x4 vs[W];
+#pragma unroll
+    for (int t = 0; t < W; ++t) {
+      const int i = min(at + t * kGroups, n - 1);
+      ls[t] = lse[i];
+      vs[t] = *reinterpret_cast<const f32x4*>(o + (int64_t)i * D);
+    }
+    float bm = mx;
+#pragma unroll
+    for (int t = 0; t < W; ++t) {
+      if (at + t * kGroups >= n) ls[t] = -INFINITY;
+      bm = fmaxf(bm, ls[t]);
+    }
+    if (bm > -INFINITY) {  // else: no partial so far saw a key for this row
+      const float a = __builtin_amdgcn_exp2f(mx - bm);
+      wsum *= a;
+      acc *= a;
+#pragma unroll
+      for (int t = 0; t < W; ++t) {
+        const float w = __builtin_amdgcn_exp2f(ls[t] - bm);
+        wsum += w;
+        acc += w * vs[t];
+      }
+      mx = bm;
+    }
+  }
+#pragma unroll
+  for (int off = kLanes; off < 64; off *= 2) {
+    const float mo = __shfl_xor(mx, off);
+    const float top = fmaxf(mx, mo);
+    const float ref = top > -INFINITY ? top : 0.f;
+    const float a = __builtin_amdgcn_exp2f(mx - ref), c = __builtin_amdgcn_exp2f(mo - ref);
+    wsum = a * wsum + c * __shfl_xor(wsum, off);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] = a * acc[e] + c * __shfl_xor(acc[e], off);
+    mx = top;
+  }
+  const bool seen = wsum > 0.f;
+  if (lane < kLanes)
+    store_row4<D>(out, sh, row, d, acc * (seen ? 1.0f / wsum : 0.f),
+                  seen ? mx + log2f(wsum) : -INFINITY);
 }
 
 // mx_lse_merge: rows merged over `parts` gathered partials, part-major ([parts, rows, D] and
