@@ -25,7 +25,8 @@
  * num_heads % num_kv_heads == 0 and num_heads / num_kv_heads <= 128; seqlen_q >= 1 with
  * batch * seqlen_q <= 65535; causal 0 or 1.  The seqlen_q * (num_heads / num_kv_heads) query
  * rows of one KV head are processed in groups of 16 rows (32 when there are more than 16 and
- * head_dim <= 128): every further group streams that head's K/V once more.
+ * head_dim <= 128): every further group streams that head's K/V once more.  Automatic plans of
+ * more rows than one group run blocks of 64 to 256 rows instead (MX_SCHEDULE_TILED).
  *
  * Every call is asynchronous on the given stream (NULL = the legacy default stream) and never
  * synchronises.  Calls that share one workspace (including the library's internal one) must
@@ -78,8 +79,10 @@ extern "C" {
                                       pairs of the batch outnumber the workgroups               */
 #define MX_SCHEDULE_TILED 4        /* blocks of 128 or 256 query rows of a KV head against K/V
                                       tiles shared through LDS, long key ranges cut into pieces
-                                      merged in the same launch: automatic plans of many query
-                                      rows per KV head                                            */
+                                      merged in the same launch (up to two) or a second one:
+                                      automatic plans of more than 32 query rows per KV head
+                                      (more than 16 at head_dim 256), where the workspace holds
+                                      its partials                                                */
 
 /* Phase flags for mx_paged_gqa_decode (0 = run everything). */
 #define MX_PHASE_MAIN_ONLY 1        /* split grid: run only the split-KV kernel, partials stay in
@@ -160,8 +163,8 @@ int mx_paged_gqa_decode(const void* q, const void* k_cache, const void* v_cache,
  * on each device when the library's code is first loaded there and holds until the process
  * ends.  The call never allocates (no hipMalloc, hipFree or allocating library routine); the
  * first call on a device also launches a clear of the array's status word and counters on
- * `stream`, ahead of its decode.  A call whose mx_paged_gqa_decode_workspace_size exceeds
- * MX_NOALLOC_SCRATCH_BYTES is rejected with MX_STATUS_UNSUPPORTED before anything is launched.
+ * `stream`, ahead of its decode.  A call whose partials exceed MX_NOALLOC_SCRATCH_BYTES on every
+ * schedule it could take (tiled plans fall back to the others) is rejected with MX_STATUS_UNSUPPORTED before anything is launched.
  * Every such call on one GPU shares that GPU's array: calls that overlap in time on one GPU
  * (different streams without ordering, or different host threads) race on it, so order them
  * on one stream.  The device status flags of these calls (a bad page id read as page 0, a

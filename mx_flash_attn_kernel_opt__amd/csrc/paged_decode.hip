@@ -3481,9 +3481,15 @@ int prepare_decode(const void* q, const void* k_cache, const void* v_cache, cons
   int st = make_plan(batch, seqlen_q, num_heads, num_kv_heads, head_dim, page_size,
                      max_pages_per_seq, max_seq_len, num_splits, 0, pair_ok, tile_ok, plan);
   if (st != MX_STATUS_OK) return st;
-  if (*workspace != nullptr && workspace_bytes < plan->workspace_bytes &&
-      plan->schedule == MX_SCHEDULE_TILED) {
-    // A workspace that holds the other schedules' partials only.
+  if (plan->schedule == MX_SCHEDULE_TILED) {
+    // The tiled partials can need more workspace than the streaming plan's.  Where they do not get
+    // it (a caller's workspace too small for them, or the library's that cannot grow: under
+    // stream capture, or out of memory), the call runs the streaming plan.
+    if (*workspace != nullptr ? workspace_bytes >= plan->workspace_bytes
+                              : internal_workspace(plan->workspace_bytes,
+                                                   static_cast<hipStream_t>(stream),
+                                                   workspace) == MX_STATUS_OK)
+      return MX_STATUS_OK;
     *plan = Plan{};
     st = make_plan(batch, seqlen_q, num_heads, num_kv_heads, head_dim, page_size,
                    max_pages_per_seq, max_seq_len, num_splits, 0, pair_ok, false, plan);

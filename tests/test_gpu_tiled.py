@@ -233,3 +233,25 @@ def test_longest_sequences_first(G, D, fp8):
         out, ref = _run(inp), _oracle(inp, False)
     assert_close_to_oracle(out, ref, f"longest first G={G} D={D}")
     assert read_device_status() == 0
+
+
+def test_capture_without_a_workspace():
+    """Captured with the library's own workspace and no call of the shape before: where that would
+    have to grow for the tiled partials, the call runs the streaming plan instead of failing."""
+    inp = _inputs([490], 4, 1, 128, 16, 480, seed=15)
+    p = _plan(inp)   # over 1 MiB of partials; the streaming plan has one split and needs none
+    assert p["schedule"] == "tiled" and p["workspace_bytes"] > 1 << 20
+    small = _inputs([40], 4, 2, 128, 16, 1, seed=16)
+    _run(small)                    # the library's workspace exists (1 MiB if nothing grew it)
+    out = torch.zeros_like(inp.q)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        _run(inp, causal=True, out=out)
+    ref = _oracle(inp, True)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_close_to_oracle(out, ref, "captured without a workspace")
+        _run(small)
