@@ -3122,6 +3122,11 @@ struct KvFormat {
   float v_scale = 1.0f;
 };
 
+// What the kernels multiply raw scores with (log2 units).
+float score_scale_log2(float scale, const KvFormat& kv) {
+  return scale * 1.4426950408889634f * (kv.fp8 ? kv.k_scale : 1.0f);
+}
+
 // KV heads as the kernels see them.  Stored heads of dim 64 run in adjacent pairs as kernel heads
 // of dim 128 (MainShape::pair_group) when a head's query rows fit one 16-row tile, so that a
 // pair is still one pass over its K/V.  For fp8 caches this is what makes the reads whole: an
@@ -3194,7 +3199,7 @@ hipError_t launch(const Plan& plan, const void* q, const void* k, const void* v,
   sh.num_pages = (num_pages > 0 && num_pages <= INT32_MAX) ? (int)num_pages : 0;
   sh.chunk_shift = plan.chunk_shift;
   sh.cap_tokens = (int)plan.cap_tokens;
-  sh.scale_log2 = scale * 1.4426950408889634f * (kv.fp8 ? kv.k_scale : 1.0f);
+  sh.scale_log2 = score_scale_log2(scale, kv);
   sh.v_scale = kv.fp8 ? kv.v_scale : 1.0f;
   sh.k_scale = kv.fp8 ? kv.k_scale : 1.0f;
   sh.num_splits = (int)plan.splits;
@@ -3464,7 +3469,8 @@ int prepare_decode(const void* q, const void* k_cache, const void* v_cache, cons
                    int64_t head_dim, int64_t page_size, int64_t num_pages,
                    int64_t max_pages_per_seq, int64_t max_seq_len, int32_t causal, float scale,
                    int64_t num_splits, void** workspace, int64_t workspace_bytes,
-                   int32_t phase, void* stream, int pair_ok, bool tile_ok, Plan* plan) {
+                   int32_t phase, void* stream, const KvFormat& kv, int pair_ok, bool tile_ok,
+                   Plan* plan) {
   if (phase != 0 && phase != MX_PHASE_MAIN_ONLY && phase != MX_PHASE_COMBINE_ONLY)
     return fail(MX_STATUS_INVALID_ARGUMENT, "phase must be 0, 1 or 2");
   // The kernels read q, K and V rows as 16-byte vectors and write out in 8-byte pieces.
@@ -3476,8 +3482,9 @@ int prepare_decode(const void* q, const void* k_cache, const void* v_cache, cons
   if (causal != 0 && causal != 1) return fail(MX_STATUS_INVALID_ARGUMENT, "causal must be 0 or 1");
   if (!std::isfinite(scale)) return fail(MX_STATUS_INVALID_ARGUMENT, "scale must be finite");
   if (num_pages < 0) return fail(MX_STATUS_INVALID_SHAPE, "num_pages must be >= 0");
-  // The tiled kernel masks unscaled scores with -inf, which a zero scale would turn into NaN.
-  tile_ok = tile_ok && fabsf(scale) >= 1e-30f;
+  // The tiled kernel masks unscaled scores with -inf, which a zero scale (of the scores: an fp8
+  // cache's k_scale is part of it) would turn into NaN.
+  tile_ok = tile_ok && fabsf(score_scale_log2(scale, kv)) >= 1e-30f;
   int st = make_plan(batch, seqlen_q, num_heads, num_kv_heads, head_dim, page_size,
                      max_pages_per_seq, max_seq_len, num_splits, 0, pair_ok, tile_ok, plan);
   if (st != MX_STATUS_OK) return st;
@@ -3557,7 +3564,7 @@ int decode_impl(const void* q, const void* k_cache, const void* v_cache, void* o
   const int st = prepare_decode(q, k_cache, v_cache, out, batch, seqlen_q, num_heads,
                                 kh.kv_heads, kh.head_dim, page_size, num_pages, max_pages_per_seq,
                                 max_seq_len, causal, scale, num_splits, &workspace,
-                                workspace_bytes, phase, stream, pair_ok_for(kv.fp8, kh),
+                                workspace_bytes, phase, stream, kv, pair_ok_for(kv.fp8, kh),
                                 /*tile_ok=*/true, &plan);
   if (st != MX_STATUS_OK) return st;
   return run_decode(plan, q, k_cache, v_cache, out, o_out, lse_out, seq_lens, block_table, batch,
@@ -3923,7 +3930,7 @@ static int decode_append_impl(const void* q, const void* k_new, const void* v_ne
   st = prepare_decode(q, k_cache, v_cache, out, batch, seqlen_q, num_heads, kh.kv_heads,
                       kh.head_dim, page_size, num_pages, max_pages_per_seq, max_seq_len, causal,
                       scale, num_splits, &workspace, workspace_bytes, 0, stream,
-                      pair_ok_for(kv.fp8, kh), /*tile_ok=*/true, &plan);
+                      kv, pair_ok_for(kv.fp8, kh), /*tile_ok=*/true, &plan);
   if (st != MX_STATUS_OK) return st;
   AppendArgs app;
   if (seqlen_new >= 1 && seqlen_new <= kChunk) {

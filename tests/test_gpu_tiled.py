@@ -111,6 +111,21 @@ def test_signs_and_zero_of_the_scale(scale):
     assert_close_to_oracle(out, ref, f"scale {scale}")
 
 
+@pytest.mark.parametrize("scale,k_scale", [(None, 0.0), (0.0, 0.5), (1e-25, 1e-25), (0.3, -0.25)])
+@pytest.mark.parametrize("D,G,sq", [(64, 8, 9), (128, 8, 9), (256, 8, 3)])
+def test_fp8_key_scales_of_zero_and_either_sign(D, G, sq, scale, k_scale):
+    """The scores' scale is scale * k_scale: where that is zero, also by underflow, a row is the
+    mean of the values it sees, masked keys (causal, and past the sequence's end) left out."""
+    inp = _inputs([1, 63, 64, 200], G, 2, D, 16, sq, seed=18)
+    assert _plan(inp, True)["schedule"] == "tiled"
+    k8, v8 = (c.to(torch.float8_e4m3fn) for c in (inp.k_cache, inp.v_cache))
+    kw = dict(k_scale=k_scale, v_scale=1.25, causal=True)
+    out = paged_gqa_decode(inp.q, k8, v8, inp.block_table, inp.seq_lens, scale, **kw)
+    ref = paged_decode_fp8_reference(inp.q.cpu(), k8.cpu(), v8.cpu(), inp.block_table.cpu(),
+                                     inp.seq_lens.cpu(), scale, **kw)
+    assert_close_to_oracle(out, ref, f"D={D} scale={scale} k_scale={k_scale}")
+
+
 def test_unused_slots_do_not_reach_the_output():
     """NaN past the sequences' ends (the rest of their last pages, and pages of no sequence)."""
     inp = _inputs([1, 33, 64, 70], 8, 2, 128, 64, 9, seed=9)
