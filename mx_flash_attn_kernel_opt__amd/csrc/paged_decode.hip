@@ -2429,18 +2429,19 @@ __global__ __launch_bounds__(256) void mx_paged_tiled_combine(
       if (at + t * kGroups >= n) ls[t] = -INFINITY;
       bm = fmaxf(bm, ls[t]);
     }
-    if (bm > -INFINITY) {  // else: no partial so far saw a key for this row
-      const float a = __builtin_amdgcn_exp2f(mx - bm);
-      wsum *= a;
-      acc *= a;
+    // (While no partial weighs anything the reference is 0, as in the merge trees: a partial with a
+    // NaN has log-sum-exp -inf, and 0 * NaN keeps the row NaN.)
+    const float ref = bm > -INFINITY ? bm : 0.f;
+    const float a = __builtin_amdgcn_exp2f(mx - ref);
+    wsum *= a;
+    acc *= a;
 #pragma unroll
-      for (int t = 0; t < W; ++t) {
-        const float w = __builtin_amdgcn_exp2f(ls[t] - bm);
-        wsum += w;
-        acc += w * vs[t];
-      }
-      mx = bm;
+    for (int t = 0; t < W; ++t) {
+      const float w = __builtin_amdgcn_exp2f(ls[t] - ref);
+      wsum += w;
+      acc += w * vs[t];
     }
+    mx = bm;
   }
 #pragma unroll
   for (int off = kLanes; off < 64; off *= 2) {

@@ -126,6 +126,40 @@ def test_fp8_key_scales_of_zero_and_either_sign(D, G, sq, scale, k_scale):
     assert_close_to_oracle(out, ref, f"D={D} scale={scale} k_scale={k_scale}")
 
 
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("L", [600, 1500, 9000])  # a few pieces, and many
+def test_nan_and_infinity_in_live_data(L, D):
+    """A row with a NaN score, or one of +inf, is NaN however its keys are cut and merged; a score
+    of -inf weighs nothing; the other rows are what they are without."""
+    sq, G = 40, 4
+    inp = _inputs([L], G, 1, D, 16, sq, seed=L + D)
+    assert _plan(inp)["schedule"] == "tiled"
+    bt, P = inp.block_table[0].long(), 16
+    q0, k0 = inp.q.clone(), inp.k_cache.clone()
+    base = _oracle(inp, True)
+
+    def check(label, bad, ref):
+        out = _run(inp, causal=True).cpu()
+        nan = out.isnan()
+        assert torch.equal(nan, bad.view(1, sq, G, 1).expand_as(nan)), label
+        if not bad.all():
+            assert_close_to_oracle(out[~nan], ref[~nan], label)
+
+    bad = torch.zeros(sq, G, dtype=torch.bool)
+    bad[3, 2] = True
+    inp.q[0, 3, 2, 5] = float("nan")
+    check(f"NaN query L={L} D={D}", bad, base)
+    inp.q.copy_(q0)
+    for t in (L // 3, L - 11):  # the second is seen by the last 11 query tokens only
+        inp.k_cache[bt[t // P], t % P, 0, 7] = float("nan")
+        sees = torch.arange(sq) + L - sq >= t
+        check(f"NaN key {t} of {L} D={D}", sees.view(sq, 1).expand(sq, G), base)
+        inp.k_cache.copy_(k0)
+    t = L // 2
+    inp.k_cache[bt[t // P], t % P, 0, 0] = float("inf")
+    check(f"infinite key {t} of {L} D={D}", inp.q[0, :, :, 0].cpu() > 0, _oracle(inp, True))
+
+
 def test_unused_slots_do_not_reach_the_output():
     """NaN past the sequences' ends (the rest of their last pages, and pages of no sequence)."""
     inp = _inputs([1, 33, 64, 70], 8, 2, 128, 64, 9, seed=9)
