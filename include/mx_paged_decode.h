@@ -252,7 +252,9 @@ int mx_lse_merge(const float* o_parts, const float* lse_parts, int64_t num_parts
  * balanced schedule), the workgroups launched and the workspace bytes a call with these
  * arguments would use.  Replaces the reference's split policy choose_num_splits
  * (submission_clean.cu:375-430) and its page-rounding of splits (submission_clean.cu:456-461).
- * num_cus <= 0 queries the current device.  Any of the out pointers may be NULL.
+ * The bytes of a tiled plan also hold the partials of the schedule that calls of the shape with a
+ * score scale below 1e-30 run instead.  num_cus <= 0 queries the current device.  Any of the out
+ * pointers may be NULL.
  */
 int mx_paged_gqa_decode_plan(int64_t batch, int64_t seqlen_q, int64_t num_heads,
                              int64_t num_kv_heads, int64_t head_dim, int64_t page_size,

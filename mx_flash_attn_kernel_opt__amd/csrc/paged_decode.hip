@@ -3401,10 +3401,20 @@ static int report_plan(bool fp8, bool tile_ok, int64_t batch, int64_t seqlen_q, 
                        int64_t* workspace_bytes_out) {
   Plan plan;
   const KernelHeads kh = kernel_heads(seqlen_q, num_heads, num_kv_heads, head_dim, fp8);
-  const int st = make_plan(batch, seqlen_q, num_heads, kh.kv_heads, kh.head_dim, page_size,
-                           max_pages_per_seq, max_seq_len, num_splits, num_cus,
-                           pair_ok_for(fp8, kh), tile_ok, &plan);
+  int st = make_plan(batch, seqlen_q, num_heads, kh.kv_heads, kh.head_dim, page_size,
+                     max_pages_per_seq, max_seq_len, num_splits, num_cus,
+                     pair_ok_for(fp8, kh), tile_ok, &plan);
   if (st != MX_STATUS_OK) return st;
+  if (plan.schedule == MX_SCHEDULE_TILED) {
+    // The bytes serve every call of the shape, also one that the tiled kernel does not take
+    // (prepare_decode): its streaming plan can need more.
+    Plan stream;
+    st = make_plan(batch, seqlen_q, num_heads, kh.kv_heads, kh.head_dim, page_size,
+                   max_pages_per_seq, max_seq_len, num_splits, num_cus, pair_ok_for(fp8, kh), false,
+                   &stream);
+    if (st != MX_STATUS_OK) return st;
+    plan.workspace_bytes = std::max(plan.workspace_bytes, stream.workspace_bytes);
+  }
   if (schedule_out) *schedule_out = plan.schedule;
   if (splits_out) *splits_out = plan.splits;
   if (tokens_per_split_out) *tokens_per_split_out = plan.tokens_per_split;

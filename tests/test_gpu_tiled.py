@@ -232,6 +232,21 @@ def test_workspace_of_the_streaming_plan_still_serves():
         _run(inp, causal=True, workspace=make_workspace(4096, DEV))
 
 
+@pytest.mark.parametrize("lens,G,D,sq", [([6000], 4, 128, 40), ([490] * 5, 40, 256, 2)])
+def test_workspace_of_the_reported_size_serves_every_scale(lens, G, D, sq):
+    """plan()'s bytes also hold the partials of the schedule that a zero scale takes."""
+    inp = _inputs(lens, G, 1, D, 16, sq, seed=17)
+    p = _plan(inp)
+    assert p["schedule"] == "tiled"
+    ws = make_workspace(p["workspace_bytes"], DEV)
+    for scale in (inp.scale, 0.0):
+        out = paged_gqa_decode(inp.q, inp.k_cache, inp.v_cache, inp.block_table, inp.seq_lens,
+                               scale, causal=True, workspace=ws)
+        ref = paged_decode_reference(inp.q.cpu(), inp.k_cache.cpu(), inp.v_cache.cpu(),
+                                     inp.block_table.cpu(), inp.seq_lens.cpu(), scale, causal=True)
+        assert_close_to_oracle(out, ref, f"scale {scale} in {p['workspace_bytes']} bytes")
+
+
 def test_bad_pages_and_long_lengths_are_flagged():
     inp = _inputs([300, 130], 8, 2, 128, 16, 8, seed=13, max_pages=20)
     bt, lens = inp.block_table.clone(), inp.seq_lens.clone()
