@@ -3259,13 +3259,13 @@ hipError_t launch(const Plan& plan, const void* q, const void* k, const void* v,
       auto pick = [&](auto wr) {
         constexpr int WR = decltype(wr)::value;
         if (kv.fp8 && append)
-          go(mx_paged_attend_tiled<D, WR, kCausal, true, true>, k8, v8);
+          go(mx_paged_attend_tiled<D, WR, true, true>, k8, v8);
         else if (kv.fp8)
-          go(mx_paged_attend_tiled<D, WR, kCausal, true, false>, k8, v8);
+          go(mx_paged_attend_tiled<D, WR, true, false>, k8, v8);
         else if (append)
-          go(mx_paged_attend_tiled<D, WR, kCausal, false, true>, k16, v16);
+          go(mx_paged_attend_tiled<D, WR, false, true>, k16, v16);
         else
-          go(mx_paged_attend_tiled<D, WR, kCausal, false, false>, k16, v16);
+          go(mx_paged_attend_tiled<D, WR, false, false>, k16, v16);
       };
       if (plan.tile_row_waves == 2)
         pick(std::integral_constant<int, 2>{});

@@ -84,7 +84,7 @@ __device__ __forceinline__ TileRange tile_range(int r0, int nrows, int seq, int 
 //    operands and spilled (head_dim 128: 276 bytes per lane, 2.3 times slower).
 
 
-template <int D, int WR, bool kCausal, bool kFp8, bool kAppend>
+template <int D, int WR, bool kFp8, bool kAppend>
 __global__ __launch_bounds__(64 * tile_waves<D>())
 __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2)))
 void mx_paged_attend_tiled(
