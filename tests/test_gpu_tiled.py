@@ -8,6 +8,10 @@ Tolerance: the package's own (max-abs <= 2e-2, mean-abs <= 2e-3 on bf16 outputs 
 
 from __future__ import annotations
 
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -214,22 +218,30 @@ def test_append_and_attend(D, P, G, S, sq, fp8):
     assert read_device_status() == 0
 
 
+# One sequence of 2 000 keys, 512 tokens of 4 heads on each of 4 KV heads: few row blocks, so the
+# tiled plan cuts them (its partials take over 8 MB), while the 256 streaming units run one split.
+SPLIT_SHAPE = dict(lens=[2000], G=4, Hkv=4, D=128, P=16, sq=512)
+
+
 def test_workspace_of_the_streaming_plan_still_serves():
     """A workspace too small for the tiled partials but not for the streaming plan's runs the
-    latter; a too small one is refused as before."""
-    inp = _inputs([6000], 4, 1, 128, 16, 40, seed=12)
-    need = _plan(inp)["workspace_bytes"]
+    latter; one too small for both is refused."""
+    inp = _inputs(**SPLIT_SHAPE, seed=12)
+    p = _plan(inp)
+    assert p["schedule"] == "tiled" and p["splits"] > 1 and p["workspace_bytes"] > 8 << 20, p
+    streaming = _run(inp, causal=True, num_splits=1).clone()
     ref = _oracle(inp, True)
-    for nbytes in (need, need - 256, 1 << 20):
-        ws = make_workspace(nbytes, DEV)
-        try:
-            out = _run(inp, causal=True, workspace=ws)
-        except _lib.MXAttnError as e:
-            assert e.status == _lib.MX_STATUS_WORKSPACE_TOO_SMALL and nbytes < need
-            continue
-        assert_close_to_oracle(out, ref, f"workspace of {nbytes} of {need} bytes")
-    with pytest.raises(_lib.MXAttnError):
-        _run(inp, causal=True, workspace=make_workspace(4096, DEV))
+    out = _run(inp, causal=True, workspace=make_workspace(p["workspace_bytes"], DEV)).clone()
+    assert not torch.equal(out, streaming)  # the tiled kernel sums in another order
+    assert_close_to_oracle(out, ref, f"workspace of {p['workspace_bytes']} bytes")
+    for nbytes in (1 << 20, 256):
+        out = _run(inp, causal=True, workspace=make_workspace(nbytes, DEV))
+        assert torch.equal(out, streaming)
+    assert_close_to_oracle(streaming, ref, "streaming plan")
+    both = _inputs([6000], 4, 1, 128, 16, 40, seed=12)  # the streaming plan has splits here
+    with pytest.raises(_lib.MXAttnError) as e:
+        _run(both, causal=True, workspace=make_workspace(4096, DEV))
+    assert e.value.status == _lib.MX_STATUS_WORKSPACE_TOO_SMALL
 
 
 @pytest.mark.parametrize("lens,G,D,sq", [([6000], 4, 128, 40), ([490] * 5, 40, 256, 2)])
@@ -299,23 +311,43 @@ def test_longest_sequences_first(G, D, fp8):
     assert read_device_status() == 0
 
 
+_CAPTURE_CHILD = """
+import torch
+from test_gpu_tiled import SPLIT_SHAPE, _inputs, _run
+
+inp, small = _inputs(**SPLIT_SHAPE, seed=15), _inputs([40], 4, 2, 128, 16, 1, seed=16)
+_run(small)                    # the library's workspace exists: 1 MiB in a process that grew none
+streaming = _run(inp, causal=True, num_splits=1).clone()
+out = torch.zeros_like(inp.q)
+torch.cuda.synchronize()
+graph = torch.cuda.CUDAGraph()
+with torch.cuda.graph(graph):
+    _run(inp, causal=True, out=out)
+for _ in range(3):
+    out.zero_()
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, streaming), "the captured call did not run the streaming plan"
+    _run(small)
+tiled = _run(inp, causal=True)  # outside the capture the workspace grows
+assert not torch.equal(tiled, streaming)
+graph.replay()                  # and the graph keeps its own
+torch.cuda.synchronize()
+assert torch.equal(out, streaming)
+print("captured without a workspace: ok", flush=True)
+"""
+
+
 def test_capture_without_a_workspace():
     """Captured with the library's own workspace and no call of the shape before: where that would
-    have to grow for the tiled partials, the call runs the streaming plan instead of failing."""
-    inp = _inputs([490], 4, 1, 128, 16, 480, seed=15)
-    p = _plan(inp)   # over 1 MiB of partials; the streaming plan has one split and needs none
-    assert p["schedule"] == "tiled" and p["workspace_bytes"] > 1 << 20
-    small = _inputs([40], 4, 2, 128, 16, 1, seed=16)
-    _run(small)                    # the library's workspace exists (1 MiB if nothing grew it)
-    out = torch.zeros_like(inp.q)
-    torch.cuda.synchronize()
-    graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
-        _run(inp, causal=True, out=out)
-    ref = _oracle(inp, True)
-    for _ in range(3):
-        out.zero_()
-        graph.replay()
-        torch.cuda.synchronize()
-        assert_close_to_oracle(out, ref, "captured without a workspace")
-        _run(small)
+    have to grow for the tiled partials, the call runs the streaming plan instead of failing.  In
+    a process of its own: the library's workspace only grows, and other tests grow it."""
+    inp = _inputs(**SPLIT_SHAPE, seed=15)
+    p = _plan(inp)
+    assert p["schedule"] == "tiled" and p["splits"] > 1 and p["workspace_bytes"] > 8 << 20, p
+    assert_close_to_oracle(_run(inp, causal=True, num_splits=1), _oracle(inp, True), "streaming")
+    tests = os.path.dirname(os.path.abspath(__file__))
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join([os.path.dirname(tests), tests]))
+    res = subprocess.run([sys.executable, "-c", _CAPTURE_CHILD], env=env, capture_output=True,
+                         text=True, timeout=100)
+    assert res.returncode == 0 and "ok" in res.stdout, res.stdout + res.stderr
