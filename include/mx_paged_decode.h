@@ -77,18 +77,20 @@ extern "C" {
                                       the batch are at least the workgroups; on bf16 caches of
                                       4 KV heads, pairs of heads 0 and 3, 1 and 2 when the
                                       pairs of the batch outnumber the workgroups               */
-#define MX_SCHEDULE_TILED 4        /* blocks of 128 or 256 query rows of a KV head against K/V
-                                      tiles shared through LDS, long key ranges cut into pieces
-                                      merged in the same launch (up to two) or a second one:
-                                      automatic plans of more than 32 query rows per KV head
-                                      (more than 16 at head_dim 256), where the workspace holds
-                                      its partials                                                */
+#define MX_SCHEDULE_TILED 4        /* blocks of 64, 128 or 256 query rows of a KV head against
+                                      K/V tiles shared through LDS, long key ranges cut into
+                                      pieces merged in the same launch (plans of up to two) or a
+                                      second one: automatic plans of more than 32 query rows per
+                                      KV head (more than 16 at head_dim 256), where the workspace
+                                      holds its partials                                          */
 
 /* Phase flags for mx_paged_gqa_decode (0 = run everything). */
 #define MX_PHASE_MAIN_ONLY 1        /* split grid: run only the split-KV kernel, partials stay in
-                                       the workspace (balanced schedule: the whole call)          */
+                                       the workspace (balanced and tiled schedules: the whole
+                                       call)                                                      */
 #define MX_PHASE_COMBINE_ONLY 2     /* split grid: run only the combine over the partials of an
-                                       identical MAIN_ONLY call (balanced schedule: nothing)      */
+                                       identical MAIN_ONLY call (balanced and tiled schedules:
+                                       nothing)                                                   */
 
 /*
  * Drop-in replacement for the reference's C500 kernel entry point, same name, argument order
@@ -136,11 +138,14 @@ void run_kernel(const void* q, const void* k_cache_paged, const void* v_cache_pa
  *                      < 0 = balanced schedule with exactly -num_splits workgroups.
  *   workspace          device memory of >= mx_paged_gqa_decode_workspace_size() bytes,
  *                      zero-filled once by the caller before first use (its first 229 632
- *                      bytes hold a status word, workgroup claim masks and merge counters
- *                      that every call leaves at zero); NULL = library-owned: one per device, grown on demand
- *                      (doubling; earlier allocations are kept, never freed, so graphs
- *                      captured with them stay valid).  A call that needs it to grow fails
- *                      with MX_STATUS_INVALID_ARGUMENT on a capturing stream.
+ *                      bytes hold a status word, a word that a tiled call's first launch
+ *                      leaves for its second, workgroup claim masks and merge counters; every
+ *                      call leaves masks and counters at zero); NULL = library-owned: one
+ *                      per device, grown on demand (doubling; earlier allocations are kept,
+ *                      never freed, so graphs captured with them stay valid).  On a capturing
+ *                      stream it cannot grow: a tiled plan then cuts into fewer pieces or runs
+ *                      on another schedule, and a call that still needs more fails with
+ *                      MX_STATUS_INVALID_ARGUMENT.
  *   phase              0, MX_PHASE_MAIN_ONLY or MX_PHASE_COMBINE_ONLY.
  *   stream             hipStream_t (NULL = legacy default stream).
  * q, k_cache and v_cache must be 16-byte aligned and out 8-byte aligned (MX_STATUS_INVALID_ARGUMENT
@@ -163,8 +168,10 @@ int mx_paged_gqa_decode(const void* q, const void* k_cache, const void* v_cache,
  * on each device when the library's code is first loaded there and holds until the process
  * ends.  The call never allocates (no hipMalloc, hipFree or allocating library routine); the
  * first call on a device also launches a clear of the array's status word and counters on
- * `stream`, ahead of its decode.  A call whose partials exceed MX_NOALLOC_SCRATCH_BYTES on every
- * schedule it could take (tiled plans fall back to the others) is rejected with MX_STATUS_UNSUPPORTED before anything is launched.
+ * `stream`, ahead of its decode.  A call whose partials on the split-grid or balanced schedule
+ * exceed MX_NOALLOC_SCRATCH_BYTES is rejected with MX_STATUS_UNSUPPORTED before anything is
+ * launched.  A tiled plan whose partials exceed it cuts into fewer pieces, or runs on one of
+ * those schedules.
  * Every such call on one GPU shares that GPU's array: calls that overlap in time on one GPU
  * (different streams without ordering, or different host threads) race on it, so order them
  * on one stream.  The device status flags of these calls (a bad page id read as page 0, a
@@ -252,8 +259,10 @@ int mx_lse_merge(const float* o_parts, const float* lse_parts, int64_t num_parts
  * balanced schedule), the workgroups launched and the workspace bytes a call with these
  * arguments would use.  Replaces the reference's split policy choose_num_splits
  * (submission_clean.cu:375-430) and its page-rounding of splits (submission_clean.cu:456-461).
- * The bytes of a tiled plan also hold the partials of the schedule that calls of the shape with a
- * score scale below 1e-30 run instead.  num_cus <= 0 queries the current device.  Any of the out
+ * A tiled plan's splits, tokens per split and workgroups are those of sequences as long as the
+ * capacity; where such pieces are long, the device cuts the batch by its lengths instead.  Its
+ * bytes also hold the partials of the schedule that calls of the shape with a score scale below
+ * 1e-30 run instead.  num_cus <= 0 queries the current device.  Any of the out
  * pointers may be NULL.
  */
 int mx_paged_gqa_decode_plan(int64_t batch, int64_t seqlen_q, int64_t num_heads,

@@ -28,8 +28,8 @@
 //    length-balanced launch that cuts the batch's chunk line into equal shares on the device
 //    and merges cut units through a fan-in-8 tree of the same kind.
 //  * Many query rows per KV head (prompt chunks, long verifications, large groups) take a third
-//    kernel, tiled.h: blocks of 64 to 256 rows against K/V tiles shared through LDS, bound by
-//    the matrix cores instead of re-reading K/V for every 16 or 32 rows.
+//    kernel, tiled.h: blocks of 64 to 256 rows against K/V tiles shared through LDS instead of
+//    re-reading K/V for every 16 or 32 rows.
 //  * Sharded decode: the same kernels can write each query row as fp32 output plus its
 //    log-sum-exp (mx_paged_gqa_decode_partial) for a cross-device merge (mx_lse_merge).
 //  * Paged K/V append (mx_paged_kv_append), and append-and-attend (mx_paged_gqa_decode_append):
@@ -611,6 +611,11 @@ struct MainShape {
   int num_slots;         // partial slots: num_groups + batch * Hkv
   // tiled schedule
   int longest_first;     // grid rows are the sequences by descending length (batch <= 512)
+  int cut_rows;          // 0, or: grid rows are the batch's pieces, cut by its lengths (cut_tiles)
+  float cut_slots_inv;   // the cut's model: 1 / workgroups that run at once, us per tile of one, us
+  float cut_tile_us;     // per piece of a cut sequence, and us for merging at all
+  float cut_merge_us;
+  float cut_fixed_us;
   // Partial outputs (sharded decode): when o_out is set, each query row is written as its fp32
   // normalised output to o_out and its natural-log sum-exp to lse_out instead of bf16 to out.
   float* o_out;
@@ -1570,7 +1575,12 @@ __device__ __forceinline__ void merge_group(const Tree& tree, int gslot, int str
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));
   const int total = nrows * (D / 4);
-  if (total > 64 * NW && W <= 16) {
+  // (Trees with blocks of many rows: as many elements as keep 32 loads of four floats in flight.)
+  constexpr int E = Tree::kElems * W <= 32 ? Tree::kElems : 32 / W;
+  if (E > 2 && total > 2 * 64 * NW) {
+    for (int e0 = tid; e0 < total; e0 += (E > 2 ? E : 2) * 64 * NW)
+      merge_elems<D, NW, W, (E > 2 ? E : 2)>(tree, e0, total, gslot, stride, gsize, final, s_lse);
+  } else if (total > 64 * NW && W <= 16) {
     for (int e0 = tid; e0 < total; e0 += 2 * 64 * NW)
       merge_elems<D, NW, W, 2>(tree, e0, total, gslot, stride, gsize, final, s_lse);
   } else {
@@ -1639,6 +1649,7 @@ __device__ __forceinline__ void merge_tree(const Tree& tree, int item, int nitem
 // the counter region holds split_groups = ceil(num_splits / kMergeFanIn) counters per unit.
 template <int D>
 struct SplitTree {
+  static constexpr int kElems = 2;
   const MainShape& sh;
   float* part_o;
   float* part_lse;
@@ -1859,6 +1870,7 @@ void mx_paged_decode_splitkv(
 // enough for 8^4 = 4096 pieces per unit), indexed like the slots.  A slot holds tile_rows rows.
 template <int D>
 struct BalancedTree {
+  static constexpr int kElems = 2;
   const MainShape& sh;
   float* part_o;
   float* part_lse;
@@ -2382,8 +2394,8 @@ __global__ __launch_bounds__(64) void mx_paged_decode_combine(
                       pair_group > 0 ? (h / pair_group) & 1 : -1);
 }
 
-// Second launch of the tiled schedule (more than kTileFusedPieces pieces): one wave per row merges
-// the pieces of the row's block of block_rows rows (tile_range, with the tiled launch's shape).  A
+// Second launch of the tiled schedule (plans of more than kTileFusedPieces pieces): one wave per row
+// merges the pieces of the row's block of block_rows rows as the tiled launch cut them.  A
 // row's D/4 16-byte pieces leave 64 / (D/4) lane groups, which take alternate partials, four at a
 // time (loads past the last re-read it and weigh nothing), and merge their sums by lane exchanges.
 // Bound by reading the partials once.  Against one wave per row with 8-byte loads in rounds of 16
@@ -2406,12 +2418,28 @@ __global__ __launch_bounds__(256) void mx_paged_tiled_combine(
   const int r0 = r / block_rows * block_rows;
   const int seq = sh.new_tokens > 0 ? seq_extent<true>(seq_lens, b, sh, status, false).keys
                                     : seq_extent<false>(seq_lens, b, sh, status, false).keys;
-  const int n = tile_range(r0, min(block_rows, sh.rows - r0), seq, kb, sh).pieces;
+  const bool cut = sh.cut_rows > 0;
+  const int per = cut ? (int)status[kTileCutWord] : sh.tokens_per_split / kb;
+  const double inv = piece_inverse(per);
+  int n = tile_pieces(block_tiles(r0, min(block_rows, sh.rows - r0), seq, kb, sh), per, inv);
+  if (!cut) n = min(n, sh.num_splits);
   if (n == 1) return;  // the main kernel wrote it
   const int64_t row = (int64_t)bt * sh.num_heads + h;
+  // Batch piece of the sequence's piece 0: after the pieces of the sequences before it.
+  int before = 0;
+  if (cut) {
+    for (int i = lane; i < b; i += 64) {
+      const int keys = sh.new_tokens > 0 ? seq_extent<true>(seq_lens, i, sh, status, false).keys
+                                         : seq_extent<false>(seq_lens, i, sh, status, false).keys;
+      before += tile_pieces(keys > 0 ? (keys + kb - 1) / kb : 0, per, inv);
+    }
+    before = __builtin_amdgcn_readlane(wave_inclusive_sum(before), 63);
+    n = min(n, sh.cut_rows - before);
+  }
+  const TileSlots slots = tile_slots(before, b, sh);
   const int d = 4 * (lane % kLanes);
-  const float* o = part_o + row * sh.num_splits * D + d;
-  const float* lse = part_lse + row * sh.num_splits;
+  const float* o = part_o + slots.at(row, 0) * D + d;
+  const float* lse = part_lse + slots.at(row, 0);
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   float wsum = 0.f, mx = -INFINITY;
   for (int at = lane / kLanes; at < n; at += W * kGroups) {
@@ -2420,8 +2448,8 @@ __global__ __launch_bounds__(256) void mx_paged_tiled_combine(
 #pragma unroll
     for (int t = 0; t < W; ++t) {
       const int i = min(at + t * kGroups, n - 1);
-      ls[t] = lse[i];
-      vs[t] = *reinterpret_cast<const f32x4*>(o + (int64_t)i * D);
+      ls[t] = lse[(int64_t)i * slots.step];
+      vs[t] = *reinterpret_cast<const f32x4*>(o + (int64_t)i * slots.step * D);
     }
     float bm = mx;
 #pragma unroll
@@ -2689,6 +2717,11 @@ struct Plan {
   int64_t row_tiles = 1;          // row groups: ceil(rows / (16 * tiles_per_group))
   int tile_row_waves = 0;         // MX_SCHEDULE_TILED: row waves per workgroup (32 rows each)
   bool longest_first = false;     // MX_SCHEDULE_TILED: sequences by descending length
+  bool cut = false;               // MX_SCHEDULE_TILED: pieces cut by the batch's lengths
+  int64_t tile_parts = 0;         // MX_SCHEDULE_TILED: batch pieces its partials hold (0: no partials)
+  int64_t cut_slots = 0;          // (MainShape)
+  double cut_tile_us = 0.;
+  double cut_merge_us = 0.;
   int tiles_per_group = 1;        // 16-row tiles one pass over K/V serves (1, or 2 above 16 rows)
   int64_t cap_tokens = 0;
   int64_t counter_offset = 0;
@@ -2957,8 +2990,6 @@ int make_stream_plan(int64_t batch, int64_t seqlen_q, int64_t num_heads, int64_t
 // rows, B=16 26.3 / 23.3, 32 rows, B=64 at 4 096 keys 172 / 110.  Far from it: 4 prompts of 1 500
 // tokens 820 / 125, a 512-token chunk over 16K keys 518 / 167.
 constexpr int64_t tile_min_rows(int64_t head_dim) { return head_dim == 256 ? 17 : 33; }
-constexpr int64_t kTileMaxPieces = 32;      // pieces of a unit's keys
-constexpr int64_t kTileMinPieceKeys = 128;  // of capacity: two tiles
 // Up to two pieces merge in the launch (the last to arrive merges a block's rows), more in a
 // second one spread over the whole device: a 512-token chunk over 16K keys in 2 pieces of 128-row
 // blocks 175 against 186 us, in 4 pieces of 256-row blocks 175 against 163.
@@ -2979,6 +3010,34 @@ int tile_row_waves(int64_t batch, int64_t num_kv_heads, int64_t rows, int64_t he
   return units8 >= num_cus || cap >= kTileLongCap ? 8 : 4;
 }
 
+// Longest modelled time of a piece that a plan cuts from its capacity; above it the pieces follow the
+// batch's lengths, for 1 to 2 us more a launch.  Decodes of 128 query heads on one KV head (us):
+// 64 sequences of 1 000-4 000 tokens, 20 us a piece 33.6 by the capacity and 34.7 by the lengths;
+// in a table of 128K tokens, 630 us a piece, 79 and 36; 256 sequences of log-uniform lengths up
+// to 8 160 143 and 66; 512 tokens over 2 000 keys in a table of 32K tokens 70 and 38.
+constexpr double kTileCutUs = 20.;
+// The combine launch, or the merge in the main one, in the model (256 tokens over 1 000 keys in 128-row
+// blocks: one piece 23.8, two merged in the launch 26.1, four in a second one 20.9).
+double tile_fixed_us(int64_t pieces) { return pieces > kTileFusedPieces ? 4. : 8.; }
+
+// A tiled plan's partials, `parts` batch pieces (no more than the batch: nothing is cut and none are
+// kept), and its workspace.
+int64_t tile_bytes(int64_t parts, int64_t batch, int64_t seq_rows, int64_t head_dim) {
+  return parts <= batch ? kStatusBytes
+                        : kPartialBase + align_up(parts * seq_rows * 4, 256) +
+                              parts * seq_rows * head_dim * 4;
+}
+void set_tile_parts(int64_t parts, int64_t batch, int64_t seq_rows, int64_t head_dim, Plan* plan) {
+  // (Merges in the launch address the partials by 32-bit offsets.)
+  parts = std::min(parts, kMaxHandoffBytes / (seq_rows * head_dim * 4));
+  plan->tile_parts = parts > batch ? parts : 0;
+  if (plan->tile_parts == 0) plan->cut = false;
+  plan->workspace_bytes = tile_bytes(parts, batch, seq_rows, head_dim);
+  plan->lse_offset = plan->tile_parts ? kPartialBase : 0;
+  plan->o_offset =
+      plan->tile_parts ? kPartialBase + align_up(plan->tile_parts * seq_rows * 4, 256) : 0;
+}
+
 // The tiled plan over a streaming plan of the same call, whose capacity it keeps.
 void plan_tiled(int64_t batch, int64_t seqlen_q, int64_t num_heads, int64_t num_kv_heads,
                 int64_t head_dim, int64_t num_cus, Plan* plan) {
@@ -2990,42 +3049,57 @@ void plan_tiled(int64_t batch, int64_t seqlen_q, int64_t num_heads, int64_t num_
   plan->tile_row_waves = wr;
   plan->row_tiles = ceil_div(plan->rows, 32 * wr);
   const int64_t units = batch * num_kv_heads * plan->row_tiles;
-  // Pieces per unit, for the shortest modelled time: rounds of workgroups, each streaming cap / n
-  // keys at the rate a workgroup measured (keys per us with every CU busy) after about 5 us of
-  // start and end, and the partials written and read back at 2 MB/us.  At most times n fills
-  // the device once (units * n <= CUs) or is 1.
   const int64_t slots = num_cus * (head_dim == 64 && wr < 8 ? 2 : 1);  // resident workgroups
+  // Keys per us that a workgroup measured with every CU busy.
   const double rate = (wr == 8 ? 33. : wr == 4 ? 52. : 68.) *
                       (head_dim == 64 ? 2. : head_dim == 128 ? 1. : 0.35);
-  // 64 rows or fewer, one block per head, and more units than run at once: the lengths decide which
-  // workgroups end last, so the longest sequences start first (64 sequences of 1 000-4 000
-  // tokens, 8 KV heads: 36 rows 167 -> 143 us, 64 rows 173 -> 148, fp8 138 -> 118).
-  plan->longest_first = wr == 2 && batch > 1 && batch <= kTileSortBatch && units > slots;
-  const int64_t row_bytes = batch * seqlen_q * num_heads * head_dim * 4;
+  // Partials are written and read back at 2 MB/us.
+  const double merge_us = (double)seqlen_q * num_heads * head_dim * 4 * 0.5e-6;
+  // Pieces that sequences as long as the capacity would be cut into, for the shortest modelled time
+  // (the device takes the same choice with the batch's lengths, cut_tiles).  Batches that fill
+  // the device twice are cut only where that gains a tenth.
   int64_t best = 1;
   double best_us = 0.;
   for (int64_t n = 1; n <= kTileMaxPieces && (n == 1 || cap >= n * kTileMinPieceKeys); ++n) {
-    const double us = ceil_div(units * n, slots) * (cap / (n * rate) + 5.) +
-                      (n > 1 ? row_bytes * n * 0.5e-6 + (n > kTileFusedPieces ? 4. : 2.) : 0.);
-    if (n == 1 || us < best_us) {
+    const double us = ceil_div(units * n, slots) * (cap / (n * rate) + kTileStartUs) +
+                      (n > 1 ? batch * n * merge_us + tile_fixed_us(n) : 0.);
+    if (n == 1 || us < (best == 1 && units >= 2 * slots ? 0.9 : 1.) * best_us) {
       best = n;
       best_us = us;
     }
   }
   const int64_t per_piece = ceil_div(cap_tiles, best);
   int64_t ns = ceil_div(cap_tiles, per_piece);
-  const int64_t prow = batch * seqlen_q * num_heads * ns;
-  if (!split_tree_fits(units, ns, prow * head_dim * 4)) ns = 1;
+  if (batch > kTileCutBatch || units * ceil_div(kTileMaxPieces, kMergeFanIn) > kMaxSlots ||
+      batch * ns * seqlen_q * num_heads * head_dim * 4 > kMaxHandoffBytes)
+    ns = 1;
   plan->splits = ns;
   plan->tokens_per_split = ns > 1 ? per_piece * kb : cap_tiles * kb;
   plan->groups = plan->slots = 0;
-  plan->lse_offset = plan->o_offset = 0;
-  plan->workspace_bytes = kStatusBytes;
-  if (ns > 1) {
-    plan->lse_offset = kPartialBase;
-    plan->o_offset = kPartialBase + align_up(prow * 4, 256);
-    plan->workspace_bytes = plan->o_offset + prow * head_dim * 4;
+  // 64 rows or fewer, one block per head, and more units than run at once: the lengths decide which
+  // workgroups end last, so the longest sequences start first (64 sequences of 1 000-4 000
+  // tokens, 8 KV heads: 36 rows 167 -> 143 us, 64 rows 173 -> 148, fp8 138 -> 118).
+  plan->longest_first = wr == 2 && batch > 1 && batch <= kTileSortBatch && units > slots;
+  // Pieces of at most tokens_per_split keys do where these take at most kTileCutUs: a batch shorter
+  // than its capacity cannot lose more.  Longer ones follow the lengths (cut_tiles), with partials
+  // for a launch of one round where the batch leaves room for it, else for a round's worth of
+  // pieces besides the sequences.  Uncut plans of more than 128 rows stay uncut (two chunks of
+  // 1 024 tokens over 2 000 and 6 000 keys 215, by the lengths 219), and so do plans that start
+  // the longest sequences first (41 ragged sequences, 48 rows, fp8: 133, by the lengths 146).
+  int64_t parts = ns * batch;
+  if (plan->tokens_per_split / rate > kTileCutUs && batch <= kTileCutBatch &&
+      !plan->longest_first && (ns > 1 || plan->rows <= 128)) {
+    plan->cut = true;
+    const int64_t round = slots / (num_kv_heads * plan->row_tiles);
+    if (batch > 1 && units < 2 * slots)
+      parts = std::max(parts, std::min({2 * batch <= round ? round : batch + round,
+                                        batch * kTileMaxPieces,
+                                        batch * (cap / kTileMinPieceKeys)}));
   }
+  plan->cut_slots = slots;
+  plan->cut_tile_us = kb / rate;
+  plan->cut_merge_us = merge_us;
+  set_tile_parts(parts, batch, seqlen_q * num_heads, head_dim, plan);
 }
 
 // The plan of a call: the streaming plan, or the tiled one where the call allows it (tile_ok) and
@@ -3243,11 +3317,17 @@ hipError_t launch(const Plan& plan, const void* q, const void* k, const void* v,
     // Rows above one pass of the streaming kernels: KT = 2, or 1 at head_dim 256 (tile_min_rows).
     if (phase == MX_PHASE_COMBINE_ONLY) return hipSuccess;  // the main phase did everything
     if constexpr (KT == (D == 256 ? 1 : 2)) {
-      sh.split_groups = (int)ceil_div(plan.splits, kMergeFanIn);
+      sh.split_groups = (int)ceil_div(kTileMaxPieces, kMergeFanIn);
       sh.fused_combine = plan.splits <= kTileFusedPieces ? 1 : 0;
       sh.longest_first = plan.longest_first ? 1 : 0;
-      const dim3 grid((unsigned)(kernel_kv * plan.row_tiles), (unsigned)batch,
-                      (unsigned)plan.splits);
+      sh.cut_rows = plan.cut ? (int)plan.tile_parts : 0;
+      sh.cut_slots_inv = 1.0f / (float)plan.cut_slots;
+      sh.cut_tile_us = (float)plan.cut_tile_us;
+      sh.cut_merge_us = (float)plan.cut_merge_us;
+      sh.cut_fixed_us = (float)tile_fixed_us(plan.splits);
+      const dim3 grid((unsigned)(kernel_kv * plan.row_tiles),
+                      (unsigned)(plan.cut ? plan.tile_parts : batch),
+                      (unsigned)(plan.cut ? 1 : plan.splits));
       auto go = [&](auto kernel, auto kc, auto vc) {
         hipLaunchKernelGGL(kernel, grid, dim3(64 * tile_waves<D>()), 0, stream, q16, kc, vc,
                            static_cast<uint16_t*>(out), seq_lens, block_table,
@@ -3500,14 +3580,24 @@ int prepare_decode(const void* q, const void* k_cache, const void* v_cache, cons
                      max_pages_per_seq, max_seq_len, num_splits, 0, pair_ok, tile_ok, plan);
   if (st != MX_STATUS_OK) return st;
   if (plan->schedule == MX_SCHEDULE_TILED) {
-    // The tiled partials can need more workspace than the streaming plan's.  Where they do not get
-    // it (a caller's workspace too small for them, or the library's that cannot grow: under
-    // stream capture, or out of memory), the call runs the streaming plan.
-    if (*workspace != nullptr ? workspace_bytes >= plan->workspace_bytes
-                              : internal_workspace(plan->workspace_bytes,
-                                                   static_cast<hipStream_t>(stream),
-                                                   workspace) == MX_STATUS_OK)
+    // The tiled partials can need more workspace than the streaming plan's.  Fewer pieces do with
+    // less (a caller's smaller workspace, or the library's that cannot grow: under stream
+    // capture, or out of memory), down to those of a batch as long as its capacity; where not even
+    // these fit, the call runs the streaming plan.
+    const int64_t seq_rows = seqlen_q * num_heads;
+    const int64_t least = tile_bytes(plan->splits * batch, batch, seq_rows, head_dim);
+    int64_t have = plan->workspace_bytes;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (*workspace != nullptr)
+      have = std::min(have, workspace_bytes);
+    else if (internal_workspace(have, s, workspace) != MX_STATUS_OK)
+      have = internal_workspace(least, s, workspace) == MX_STATUS_OK ? least : 0;
+    if (have >= least) {
+      int64_t parts = plan->tile_parts;
+      while (parts > batch && tile_bytes(parts, batch, seq_rows, head_dim) > have) --parts;
+      set_tile_parts(parts, batch, seq_rows, head_dim, plan);
       return MX_STATUS_OK;
+    }
     *plan = Plan{};
     st = make_plan(batch, seqlen_q, num_heads, num_kv_heads, head_dim, page_size,
                    max_pages_per_seq, max_seq_len, num_splits, 0, pair_ok, false, plan);

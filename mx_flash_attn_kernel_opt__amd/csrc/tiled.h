@@ -12,8 +12,15 @@ constexpr int tile_waves() {
 }
 constexpr int tile_keys_of(int64_t head_dim, int wr) { return head_dim == 256 || wr == 2 ? 32 : 64; }
 
-// Largest batch ordered by length (MainShape::longest_first).
+// Largest batch ordered by length (MainShape::longest_first), and cut by its lengths (cut_tiles).
 constexpr int kTileSortBatch = 512;
+constexpr int kTileCutBatch = 1024;
+constexpr int kTileMaxPieces = 32;      // pieces of the longest sequence
+constexpr int kTileMinPieceKeys = 128;  // two tiles
+constexpr float kTileStartUs = 5.f;     // start and end of a workgroup in the cut's model
+// Word of the workspace's status region in which a cut launch leaves its tiles per piece for the
+// combine kernel behind it.
+constexpr int kTileCutWord = 8;
 
 // One 16-byte LDS segment of a tile row from the 8 elements a lane loaded.
 __device__ __forceinline__ u32x4 tile_segment(u32x4 x) { return x; }
@@ -42,35 +49,218 @@ __device__ __forceinline__ float pair_sum(float x) {
   return as_float(a[0]) + as_float(a[1]);
 }
 
-// Key range of row block [r0, r0 + nrows) of a sequence of `seq` keys: the tiles of KB keys its
-// last row sees, and the equal pieces they are cut into (at most sh.num_splits, each of at most
-// sh.tokens_per_split keys).
-struct TileRange {
-  int tiles;
-  int pieces;
-};
-__device__ __forceinline__ TileRange tile_range(int r0, int nrows, int seq, int kb,
-                                                const MainShape& sh) {
+// Tiles of KB keys that row block [r0, r0 + nrows) of a sequence of `seq` keys sees.
+__device__ __forceinline__ int block_tiles(int r0, int nrows, int seq, int kb,
+                                           const MainShape& sh) {
   const int top = min(seq, row_key_limit(r0 + nrows - 1, seq, sh));
-  const int nt = top > 0 ? (top + kb - 1) / kb : 0;
-  const int per_piece = sh.tokens_per_split / kb;
-  return TileRange{nt, max(1, min(sh.num_splits, (nt + per_piece - 1) / per_piece))};
+  return top > 0 ? (top + kb - 1) / kb : 0;
 }
 
-// Grid (KV heads * row blocks, batch, pieces); see plan_tiled for the shape.  A workgroup holds 32*WR
+// Pieces of a sequence or row block of `tiles` tiles, at most `per` (inv = 1.0 / per) each.
+__device__ __forceinline__ int tile_pieces(int tiles, int per, double inv) {
+  return max(1, div_floor(tiles + per - 1, inv));
+}
+
+// Modelled time (us) of a launch of `count` workgroups over `slots` resident ones, the longest of
+// which takes `longest` and all of which take `total`: rounds of the longest, or a list of unequal
+// ones that ends at most one workgroup after the mean, whichever is less.
+__device__ __forceinline__ float tile_launch_us(float count, float slots_inv, float longest,
+                                                float total) {
+  const float rounds = ceilf(count * slots_inv - 1e-3f);  // (a full round's product may exceed 1)
+  return fminf(rounds * longest, total * slots_inv + longest);
+}
+
+// How a batch is cut (MainShape::cut_rows > 0), from its lengths alone and not from the capacity, which
+// is the block table's width and often far beyond them: the longest sequence into n
+// pieces, every other one into pieces of at most that many tiles, for the n of 1 .. kTileMaxPieces
+// whose modelled time is shortest among those with at most cut_rows pieces in the batch and, if
+// n > 1, at least kTileMinPieceKeys keys in one.  Grid row y is the batch's y-th piece.
+struct TileCut {
+  int b;      // sequence, or -1: the batch has no piece y
+  int piece;  // of the sequence
+  int per;    // tiles per piece
+  int len;    // the sequence's seq_lens entry
+};
+
+// max / unsigned min over the 64 lanes of a wave (x >= 0), in every lane (cf. wave_inclusive_sum).
+#define MX_WAVE_FOLD(OP, ID)                                                                    \
+  x = OP(x, (decltype(x))__builtin_amdgcn_update_dpp(ID, (int)x, 0x111, 0xf, 0xf, false));      \
+  x = OP(x, (decltype(x))__builtin_amdgcn_update_dpp(ID, (int)x, 0x112, 0xf, 0xf, false));      \
+  x = OP(x, (decltype(x))__builtin_amdgcn_update_dpp(ID, (int)x, 0x114, 0xf, 0xf, false));      \
+  x = OP(x, (decltype(x))__builtin_amdgcn_update_dpp(ID, (int)x, 0x118, 0xf, 0xf, false));      \
+  x = OP(x, (decltype(x))__builtin_amdgcn_update_dpp(ID, (int)x, 0x142, 0xa, 0xf, false));      \
+  x = OP(x, (decltype(x))__builtin_amdgcn_update_dpp(ID, (int)x, 0x143, 0xc, 0xf, false));      \
+  return (decltype(x))__builtin_amdgcn_readlane((int)x, 63)
+__device__ __forceinline__ int wave_max(int x) { MX_WAVE_FOLD(max, 0); }
+__device__ __forceinline__ uint32_t wave_min(uint32_t x) { MX_WAVE_FOLD(min, -1); }
+#undef MX_WAVE_FOLD
+
+// Close enough to 1.0 / d for div_floor on tile counts (below 2^27): the reciprocal's approximation
+// and one Newton step.
+__device__ __forceinline__ double piece_inverse(int d) {
+  const double r = __builtin_amdgcn_rcp((double)d);
+  return r * (2.0 - d * r);
+}
+
+// Every thread of the workgroup calls it, for a batch of at most 64 * kEach: lane l of every wave
+// holds the lengths of sequences l * kEach on.  The waves count the pieces of the batch for some n
+// each (s_count: kTileMaxPieces words of LDS that the caller does not write before its next
+// barrier), then every wave models all n, a lane each, and finds y by a prefix sum.
+template <int NW, bool kAppend, int kEach>
+__device__ __forceinline__ TileCut cut_tiles_of(const int32_t* __restrict__ seq_lens, int y, int kb,
+                                                const MainShape& sh, uint32_t* s_count) {
+  constexpr int G = kTileMaxPieces / NW;  // candidates per wave
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int b0 = lane * kEach;
+  int len[kEach], tiles[kEach];
+#pragma unroll
+  for (int i = 0; i < kEach; ++i) len[i] = seq_lens[min(b0 + i, sh.batch - 1)];
+  int top = 0, sum = 0;
+#pragma unroll
+  for (int i = 0; i < kEach; ++i) {
+    const int keys = seq_extent_of<kAppend>(len[i], sh, nullptr, false).keys;
+    tiles[i] = keys > 0 && b0 + i < sh.batch ? (keys + kb - 1) / kb : 0;
+    top = max(top, tiles[i]);
+    sum += tiles[i];
+  }
+  top = wave_max(top);
+  const float total = __builtin_amdgcn_readlane(wave_inclusive_sum(sum), 63);
+  // Pieces of this lane's sequences, those of sequences in one piece in the low half.
+  auto count = [&](int per, double inv) {
+    uint32_t c = 0;
+#pragma unroll
+    for (int i = 0; i < kEach; ++i) {
+      const int np = tile_pieces(tiles[i], per, inv);
+      if (b0 + i < sh.batch) c += np > 1 ? (uint32_t)np << 16 : 1u;
+    }
+    return c;
+  };
+  const int n = lane % kTileMaxPieces + 1;  // this lane's candidate
+  int per = max(1, div_floor(top + n - 1, piece_inverse(n)));
+  uint32_t c;
+  if (sh.batch == 1) {
+    const int np = tile_pieces(top, per, piece_inverse(per));
+    c = np > 1 ? (uint32_t)np << 16 : 1u;
+  } else {
+#pragma unroll
+    for (int k = 0; k < G; ++k) {
+      const int pk = __builtin_amdgcn_readlane(per, wv * G + k);
+      const uint32_t sum_k = wave_inclusive_sum((int)count(pk, piece_inverse(pk)));
+      if (lane == 63) s_count[wv * G + k] = sum_k;
+    }
+    __syncthreads();
+    c = s_count[n - 1];
+  }
+  const float cut = c >> 16, pieces = cut + (c & 0xffff);
+  const float wgs = gridDim.x;  // per piece
+  const float us =
+      tile_launch_us(pieces * wgs, sh.cut_slots_inv, per * sh.cut_tile_us + kTileStartUs,
+                     (total * sh.cut_tile_us + pieces * kTileStartUs) * wgs) +
+      (n > 1 ? cut * sh.cut_merge_us + sh.cut_fixed_us : 0.f);
+  const bool ok = n == 1 || (pieces <= sh.cut_rows && top * kb >= n * kTileMinPieceKeys);
+  // (Positive floats order as their bits do; n in the low ones, the least of equal times.)
+  const uint32_t best =
+      wave_min((as_u32(ok ? fmaxf(us, 0.f) : INFINITY) & ~(kTileMaxPieces - 1u)) + (uint32_t)(n - 1));
+  per = __builtin_amdgcn_readlane(per, best % kTileMaxPieces);
+  const double inv = piece_inverse(per);
+  const uint32_t mine2 = count(per, inv);
+  const int mine = (int)((mine2 >> 16) + (mine2 & 0xffff));
+  const int first = wave_inclusive_sum(mine) - mine;
+  const uint64_t holds = __builtin_amdgcn_ballot_w64(first <= y && y < first + mine);
+  if (holds == 0) return TileCut{-1, 0, per, 0};
+  int i0 = 0, piece = y - first, at = len[0];  // (in the lane that holds y)
+#pragma unroll
+  for (int i = 0; i + 1 < kEach; ++i) {
+    const int np = tile_pieces(tiles[i], per, inv);
+    if (i0 == i && piece >= np) {
+      piece -= np;
+      i0 = i + 1;
+      at = len[i + 1];
+    }
+  }
+  const int src = __builtin_ctzll(holds);
+  return TileCut{__builtin_amdgcn_readlane(b0 + i0, src), __builtin_amdgcn_readlane(piece, src),
+                 per, __builtin_amdgcn_readlane(at, src)};
+}
+
+// Bound by its chain of dependent steps, which every workgroup of a cut launch goes through before
+// its first load of K: 1 to 2 us for up to 64 sequences, so few steps and no unused code in them (a
+// loop over the lengths in LDS took 0.5 us more, and 2 more for 256 sequences).
+template <int NW, bool kAppend>
+__device__ __forceinline__ TileCut cut_tiles(const int32_t* __restrict__ seq_lens, int y, int kb,
+                                             const MainShape& sh, uint32_t* s_count) {
+  static_assert(kTileCutBatch == 64 * 16, "the widest form holds the largest batch");
+  if (sh.batch <= 64) return cut_tiles_of<NW, kAppend, 1>(seq_lens, y, kb, sh, s_count);
+  if (sh.batch <= 256) return cut_tiles_of<NW, kAppend, 4>(seq_lens, y, kb, sh, s_count);
+  return cut_tiles_of<NW, kAppend, 16>(seq_lens, y, kb, sh, s_count);
+}
+
+// Partials of the tiled launch: one fp32 output row and log2-sum-exp per (query row, piece of its
+// sequence).  Pieces of a fixed length: num_splits of every row side by side.  Pieces that follow
+// the lengths: the batch's pieces one after another, each with its sequence's rows.
+struct TileSlots {
+  int64_t mul, add;  // slot of (row, piece): row * mul + add + piece * step
+  int step;
+  __device__ __forceinline__ int64_t at(int64_t row, int piece) const {
+    return row * mul + add + (int64_t)piece * step;
+  }
+};
+// `first`: the batch piece that is sequence b's piece 0.
+__device__ __forceinline__ TileSlots tile_slots(int first, int b, const MainShape& sh) {
+  if (sh.cut_rows == 0) return TileSlots{sh.num_splits, 0, 1};
+  const int seq_rows = sh.seqlen_q * sh.num_heads;
+  return TileSlots{1, (int64_t)(first - b) * seq_rows, seq_rows};
+}
+
+// The merge tree over the pieces of a row block (merge_tree).  A block has up to 256 rows for its
+// threads and few pieces: a thread merges up to kElems elements per round trip (two pieces of
+// 128-row blocks, 256 tokens over 1 000 keys: 28.4 -> 26.0 us a call against 2 elements).
+template <int D>
+struct TileTree {
+  // (head_dim 64 has 128 registers at most; at 256 the merge's would cost the main loop.)
+  static constexpr int kElems = D == 128 ? 8 : 2;
+  const MainShape& sh;
+  float* part_o;
+  float* part_lse;
+  uint32_t* counters;
+  uint16_t* out;
+  int64_t rbase;  // row_base of the unit
+  TileSlots slots;
+  int kv;
+  int r0;
+  int unit;       // (sequence, KV head and row block) index
+  __device__ __forceinline__ int64_t at(int hh, int slot) const {
+    return slots.at(rbase + row_offset(kv, r0 + hh, sh), slot);
+  }
+  __device__ __forceinline__ float* o(int hh, int slot) const { return part_o + at(hh, slot) * D; }
+  __device__ __forceinline__ float* lse(int hh, int slot) const { return part_lse + at(hh, slot); }
+  __device__ __forceinline__ uint32_t* counter(int level, int slot) const {
+    return counters + (int64_t)level * kMaxSlots + (int64_t)unit * sh.split_groups +
+           slot / kMergeFanIn;
+  }
+  __device__ __forceinline__ int lse_step() const { return slots.step; }
+  __device__ __forceinline__ int o_step() const { return slots.step * D; }
+  __device__ __forceinline__ void store(int hh, int d, f32x4 v, float l) const {
+    store_row4<D>(out, sh, rbase + row_offset(kv, r0 + hh, sh), d, v, l);
+  }
+};
+
+// Grid (KV heads * row blocks, batch), or (KV heads * row blocks, cut_rows) where the batch is cut
+// into pieces by its lengths (cut_tiles); see plan_tiled for the shape.  A workgroup holds 32*WR
 // query rows of one (sequence, KV head) and streams one piece of their keys in tiles of KB.
 //
 // What bounds it: with many rows per head the work is two matrix products, 4 * D flop per row and
 // key, so K and V are read once per 32*WR rows (the streaming kernels: per 16 or 32) and shared
 // through LDS.  A 4 096-token prompt (Hq=32, Hkv=8, D=128) runs at 970 TFLOP/s of bf16 MFMA,
 // where a large library product reaches 1 240-1 360 on the same card; the streaming kernels ran
-// it at 135.  Per tile of 64 keys a wave issues 32 MFMAs (1 024 cycles) and about 150 VALU
+// it at 135.  Per tile of 64 keys a wave issues 32 MFMAs (1 024 cycles) and 180 other VALU
 // instructions, LDS serves 8 waves x 32 KB at up to 256 bytes per cycle, and two waves per SIMD
 // (210-230 registers at head_dim 128) cover each other's softmax and waits.
 //
 //  * QK is S^T = K . Q^T in 32x32x16 MFMAs: the result leaves lane (row r32, half hi) the scores of
 //    keys 4*hi + {0..3, 8..11, 16..19, 24..27} of its own query row, so the row maximum is 31
-//    in-lane steps and one lane swap.
+//    in-lane steps (15 in tiles of 32 keys) and one lane swap.
 //  * PV is O^T = V^T . P^T with P straight from those registers: the contraction's key order is free,
 //    so V^T is read in the order P has (ds_read_b64_tr_b16 transposes 4 keys x 16 dims per 16
 //    lanes), and P never moves.  Both operands are rounded exactly as in the streaming kernels.
@@ -82,11 +272,12 @@ __device__ __forceinline__ TileRange tile_range(int r0, int nrows, int seq, int 
 //    sequence's end are stored to LDS as zero V.  A wave skips tiles past its rows' last key.
 //  * One code path for masked and full tiles: instantiated twice, the compiler hoisted both tiles'
 //    operands and spilled (head_dim 128: 276 bytes per lane, 2.3 times slower).
-
+//  * Scratch: 20 bytes a lane at head_dim 256 with a fused bf16 append in 64-row blocks, outside the
+//    tile loop; none in the others.
 
 template <int D, int WR, bool kFp8, bool kAppend>
 __global__ __launch_bounds__(64 * tile_waves<D>())
-__attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2)))
+__attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : D == 64 && WR == 2 ? 4 : 2)))
 void mx_paged_attend_tiled(
     const uint16_t* __restrict__ q, CachePtr<kAppend, CacheElem<kFp8>> kc,
     CachePtr<kAppend, CacheElem<kFp8>> vc, uint16_t* __restrict__ out,
@@ -148,13 +339,29 @@ void mx_paged_attend_tiled(
   }
   const int r0 = blk * RB;
   const int nrows = min(RB, sh.rows - r0);
+  int piece = blockIdx.z, per = sh.tokens_per_split / KB, len;
+  int first = 0;  // batch piece of the sequence's piece 0
+  if (sh.cut_rows > 0) {
+    const TileCut cut =
+        cut_tiles<NW, kAppend>(seq_lens, b, KB, sh, reinterpret_cast<uint32_t*>(s_lse));
+    if (blockIdx.x == 0 && b == 0 && tid == 0) status[kTileCutWord] = cut.per;
+    if (cut.b < 0) return;
+    piece = cut.piece;
+    per = cut.per;
+    len = cut.len;
+    first = b - piece;
+    b = cut.b;
+    __syncthreads();  // (s_lse)
+  } else {
+    len = seq_lens[b];
+  }
 
-  const SeqExtent ext = seq_extent<kAppend>(seq_lens, b, sh, status,
-                                            blockIdx.z == 0 && blockIdx.x == 0 && tid == 0);
+  const SeqExtent ext = seq_extent_of<kAppend>(len, sh, status,
+                                               piece == 0 && blockIdx.x == 0 && tid == 0);
   const int seq = ext.keys;
-  const TileRange range = tile_range(r0, nrows, seq, KB, sh);
-  const int nt = range.tiles, np = range.pieces;
-  const int piece = blockIdx.z;
+  const int nt = block_tiles(r0, nrows, seq, KB, sh);
+  int np = tile_pieces(nt, per, piece_inverse(per));
+  if (sh.cut_rows == 0) np = min(np, sh.num_splits);
   if (piece >= np) return;
   const int64_t rbase = row_base(b, kv, sh);
   if (nt == 0) {
@@ -429,6 +636,8 @@ void mx_paged_attend_tiled(
   if constexpr (kFp8) inv *= sh.v_scale;
   const float lse = seen ? m + log2f(l) : -INFINITY;
   const int64_t row = rbase + row_offset(kv, live ? r : 0, sh);
+  const TileSlots slots = tile_slots(first, b, sh);
+  const int64_t prow = slots.at(row, piece);
   if (live && wk == 0) {
 #pragma unroll
     for (int i = 0; i < D / 32; ++i)
@@ -439,19 +648,19 @@ void mx_paged_attend_tiled(
         if (np == 1)
           store_row4<D>(out, sh, row, d, v, lse);
         else if (sh.fused_combine)
-          store_partial4(part_o, part_o + (row * sh.num_splits + piece) * D + d, v);
+          store_partial4(part_o, part_o + prow * D + d, v);
         else
-          *reinterpret_cast<f32x4*>(part_o + (row * sh.num_splits + piece) * D + d) = v;
+          *reinterpret_cast<f32x4*>(part_o + prow * D + d) = v;
       }
     if (np > 1 && hi == 0) {
       if (sh.fused_combine)
-        store_partial1(part_lse + row * sh.num_splits + piece, lse);
+        store_partial1(part_lse + prow, lse);
       else
-        part_lse[row * sh.num_splits + piece] = lse;
+        part_lse[prow] = lse;
     }
   }
   if (np == 1 || !sh.fused_combine) return;
-  const SplitTree<D> tree{sh,  part_o, part_lse, counters, out, rbase, kv, r0,
-                          b * (int)gridDim.x + (int)blockIdx.x};
+  const TileTree<D> tree{sh, part_o, part_lse, counters, out, rbase, slots, kv, r0,
+                         b * (int)gridDim.x + (int)blockIdx.x};
   merge_tree<D, NW, kMergeFanIn>(tree, piece, np, nrows, s_lse, &s_last);
 }

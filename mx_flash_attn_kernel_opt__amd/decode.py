@@ -74,8 +74,10 @@ def plan(batch: int, num_heads: int, num_kv_heads: int, head_dim: int, page_size
 
     Returns ``{"schedule", "splits", "tokens_per_split", "workgroups", "workspace_bytes",
     "launches"}`` (schedule: "split_grid", "balanced", either with "_paired": adjacent KV
-    heads in pairs, or "tiled": many query rows per KV head; launches: kernels a phase-0 call
-    runs); raises MXAttnError for an invalid or unsupported shape.
+    heads in pairs, or "tiled": many query rows per KV head, whose splits, tokens and workgroups
+    are those of sequences as long as the capacity, while a call may cut by its lengths instead;
+    launches: kernels a phase-0 call runs); raises MXAttnError for an invalid or unsupported
+    shape.
     """
     lib = _lib.load()
     sch, ns, tps, wgs, ws = (ctypes.c_int64() for _ in range(5))

@@ -311,6 +311,140 @@ def test_longest_sequences_first(G, D, fp8):
     assert read_device_status() == 0
 
 
+def _wide(inp, tokens=1 << 17):
+    """The table of a pool for long contexts: columns past the lengths name no page (reading one is
+    flagged), and the plan's capacity is far from the lengths."""
+    t = torch.full((inp.spec.batch, tokens // inp.spec.page_size), 1 << 30, dtype=torch.int32,
+                   device=DEV)
+    for b, n in enumerate(inp.seq_lens.tolist()):
+        used = -(-max(n, 0) // inp.spec.page_size)
+        t[b, :used] = inp.block_table[b, :used]
+    return t
+
+
+@pytest.mark.parametrize("G,sq", [(65, 1), (3, 43), (1, 256), (4, 129)])
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("tokens,fp8", [(2304, True), (8192, False)])
+def test_row_blocks_under_long_capacities(tokens, fp8, D, G, sq):
+    """Blocks of 128 rows (capacities of 1 025 to 4 095 tokens, and head_dim 256) and of 256 at the
+    tile edges, in pieces and whole."""
+    inp = _inputs(LENS, G, 2, D, 16, sq, seed=G + sq + D)
+    bt, s, causal = _wide(inp, tokens), inp.spec, sq > 1
+    p = plan(s.batch, s.num_heads, 2, D, 16, bt.shape[1], seqlen_q=sq, fp8=fp8)
+    rows = 256 if D < 256 and tokens >= 4096 and G * sq > 128 else 128
+    assert p["workgroups"] == 20 * -(-G * sq // rows) * p["splits"], p
+    label = f"D={D} G={G} sq={sq} capacity {tokens} fp8={fp8} {p}"
+    print(label, flush=True)
+    kw = dict(causal=causal)
+    k, v, ref = inp.k_cache, inp.v_cache, None
+    if fp8:
+        kw.update(k_scale=0.75, v_scale=1.25)
+        k, v = k.to(torch.float8_e4m3fn), v.to(torch.float8_e4m3fn)
+        ref = paged_decode_fp8_reference(inp.q.cpu(), k.cpu(), v.cpu(), inp.block_table.cpu(),
+                                         inp.seq_lens.cpu(), inp.scale, **kw)
+    else:
+        ref = _oracle(inp, causal)
+    out = paged_gqa_decode(inp.q, k, v, bt, inp.seq_lens, inp.scale, **kw)
+    assert_close_to_oracle(out, ref, label)
+    assert torch.equal(out, paged_gqa_decode(inp.q, k, v, bt, inp.seq_lens, inp.scale, **kw))
+    assert read_device_status() == 0
+
+
+CUT_WORD = 8  # kTileCutWord: tiles per piece of the last cut launch
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("lens,G,Hkv,sq,fp8", [
+    ([2100], 4, 2, 40, False),                          # one sequence: no counting of the batch
+    ([1500, 0, 33, -3, 700], 8, 2, 17, True),           # merged in the second launch
+    ([1900] + [1 + 7 * i for i in range(63)], 33, 1, 1, False),   # a sequence per lane ...
+    ([5, 1900] + [1 + 7 * i for i in range(63)], 64, 1, 1, False),  # ... and four
+    ([(97 * i) % 230 for i in range(255)] + [1800], 33, 1, 1, True),
+    ([1800] + [(97 * i) % 230 for i in range(256)], 80, 1, 1, False),  # ... and sixteen
+    ([900, 2000] * 35, 9, 1, 5, False),                 # most sequences in several pieces
+])
+def test_pieces_follow_the_lengths(lens, G, Hkv, sq, fp8, D):
+    """A batch far shorter than its table is cut by its own lengths: several pieces of the longest
+    sequence, each key in one of them, whichever workgroups merge, on less workspace too."""
+    inp = _inputs([max(n, 0) for n in lens], G, Hkv, D, 16, sq, seed=len(lens) + D)
+    inp.seq_lens.copy_(torch.tensor(lens, dtype=torch.int32))
+    bt, causal = _wide(inp), sq > 1
+    s = inp.spec
+    p = plan(s.batch, s.num_heads, Hkv, D, 16, bt.shape[1], seqlen_q=sq, fp8=fp8)
+    assert p["schedule"] == "tiled", p
+    label = f"cut B={s.batch} D={D} G={G} sq={sq} fp8={fp8}"
+    print(label, flush=True)
+    kw = dict(causal=causal)
+    lens_cpu = inp.seq_lens.cpu()
+    if fp8:
+        kw.update(k_scale=0.75, v_scale=1.25)
+        k, v = (c.to(torch.float8_e4m3fn) for c in (inp.k_cache, inp.v_cache))
+        ref = paged_decode_fp8_reference(inp.q.cpu(), k.cpu(), v.cpu(), inp.block_table.cpu(),
+                                         lens_cpu, inp.scale, **kw)
+    else:
+        k, v = inp.k_cache, inp.v_cache
+        ref = _oracle(inp, causal)
+    run = lambda **more: paged_gqa_decode(inp.q, k, v, bt, inp.seq_lens, inp.scale,  # noqa: E731
+                                          **kw, **more)
+    ws = make_workspace(p["workspace_bytes"], DEV)
+    out = run(workspace=ws).clone()
+    assert_close_to_oracle(out, ref, label)
+    per = ws.view(torch.int32)[CUT_WORD].item()
+    assert 2 <= per < max(lens) // 32, (per, p)  # tiles of 32 keys or more
+    for _ in range(3):
+        assert torch.equal(run(workspace=ws), out)
+    assert not ws[256:256 + 4096].any().item()  # no claim words in a tiled launch
+    assert read_device_status(ws) == 0
+    if p["splits"] > 1:  # the partials of a batch as long as the table, and no more
+        least = s.batch * p["splits"] * sq * s.num_heads * (D + 1) * 4 + (1 << 20)
+        if least < p["workspace_bytes"]:
+            assert_close_to_oracle(run(workspace=make_workspace(least, DEV)), ref, "less " + label)
+    elif p["launches"] == 1:  # a batch that need not be cut: any workspace serves it
+        assert_close_to_oracle(run(workspace=make_workspace(256, DEV)), ref, "uncut " + label)
+    if not fp8:
+        o, _ = paged_gqa_decode_partial(inp.q, k, v, bt, inp.seq_lens, inp.scale, causal=causal)
+        assert_close_to_oracle(o.to(torch.bfloat16), ref, "partial " + label)
+
+
+@pytest.mark.parametrize("D,S,sq,fp8", [(128, 9, 9, False), (128, 40, 40, True), (64, 16, 12, True),
+                                        (256, 3, 5, False), (256, 16, 20, True)])
+def test_append_with_pieces_that_follow_the_lengths(D, S, sq, fp8):
+    """New tokens in a cut launch: attended once and written once (by piece 0)."""
+    lens, Hkv, G, P = [1500, 0, 31, -2, 400], 2, 8, 16
+    B, need = len(lens), (1500 + S) // P + 1
+    g = torch.Generator().manual_seed(S + D)
+    mk = lambda *shape: torch.randn(*shape, generator=g).to(torch.bfloat16)  # noqa: E731
+    k, v = mk(B * need, P, Hkv, D), mk(B * need, P, Hkv, D)
+    table = torch.full((B, 8192), 1 << 30, dtype=torch.int32)
+    perm = torch.randperm(B * need, generator=g).to(torch.int32).view(B, need)
+    for b, n in enumerate(lens):
+        table[b, :-(-(max(n, 0) + S) // P)] = perm[b, :-(-(max(n, 0) + S) // P)]
+    kn, vn, q = mk(B, S, Hkv, D), mk(B, S, Hkv, D), mk(B, sq, G * Hkv, D)
+    lens_t = torch.tensor(lens, dtype=torch.int32)
+    assert plan(B, G * Hkv, Hkv, D, P, 8192, seqlen_q=sq, fp8=fp8)["schedule"] == "tiled"
+    label = f"cut append D={D} S={S} sq={sq} fp8={fp8}"
+    print(label, flush=True)
+    kw = {}
+    if fp8:
+        kw = dict(k_scale=0.75, v_scale=1.25)
+        k, v = k.to(torch.float8_e4m3fn), v.to(torch.float8_e4m3fn)
+        k2, v2, flags = paged_kv_append_reference(kn, vn, k, v, table, lens_t, **kw)
+        ref = paged_decode_fp8_reference(q, k2, v2, table, lens_t.clamp(min=0) + S, causal=True,
+                                         **kw)
+    else:
+        ref, k2, v2, flags = paged_decode_append_reference(q, kn, vn, k, v, table, lens_t,
+                                                           causal=True)
+    assert not flags
+    kd, vd = k.to(DEV), v.to(DEV)
+    out = paged_gqa_decode_append(q.to(DEV), kn.to(DEV), vn.to(DEV), kd, vd, table.to(DEV),
+                                  lens_t.to(DEV), causal=True, **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(kd.cpu().view(torch.uint8), k2.view(torch.uint8))
+    assert torch.equal(vd.cpu().view(torch.uint8), v2.view(torch.uint8))
+    assert_close_to_oracle(out, ref, label)
+    assert read_device_status() == 0
+
+
 _CAPTURE_CHILD = """
 import torch
 from test_gpu_tiled import SPLIT_SHAPE, _inputs, _run

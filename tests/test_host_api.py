@@ -623,6 +623,20 @@ def test_tiled_plan_block_rows_and_pieces(B, Hq, Hkv, D, sq, cap, rows, pieces):
     assert p["launches"] == (2 if pieces > 2 else 1)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,D,sq", [(16, 128, 1, 128, 1), (64, 128, 1, 128, 1),
+                                           (8, 32, 8, 128, 16), (1, 32, 8, 128, 512),
+                                           (256, 128, 1, 128, 1), (16, 16, 2, 256, 4)])
+def test_tiled_workspace_does_not_follow_the_table(B, Hq, Hkv, D, sq):
+    """Partials of at most 32 pieces a sequence, whatever the capacity, and of a round of workgroups
+    besides the sequences for ragged batches."""
+    row = sq * Hq * (D + 1) * 4
+    base = 229632 + 256
+    for width in (256, 2048, 8192, 65536):
+        p = plan(B, Hq, Hkv, D, 16, width, num_cus=256, seqlen_q=sq)
+        assert p["schedule"] == "tiled" and p["splits"] <= 32
+        assert p["workspace_bytes"] <= base + max(B * p["splits"], B + 256) * row, (width, p)
+
+
 @pytest.mark.parametrize("D,first", [(64, 33), (128, 33), (256, 17)])
 def test_tiled_plan_starts_above_one_streaming_pass(D, first):
     """Rows that one pass of a streaming kernel serves stay on it, and so do explicit split and
