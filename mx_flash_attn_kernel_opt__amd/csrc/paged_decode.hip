@@ -3001,10 +3001,19 @@ constexpr int64_t kTileFusedPieces = 2;
 // keys 163 / 175 / 230), and lose on the rest (1 prompt of 1 000 tokens 40 / 31 / 33; 512 tokens
 // over 2K keys 47.5 / 46.4 / 43.9; 64 tokens over 8K keys 31.6 / 29.4 / 30.4, each at its best
 // piece count).  At head_dim 256 a wave takes a SIMD's registers: four waves, two or four on rows.
+//
+// Up to half a round of 128-row blocks over short keys takes 64-row blocks, which leave fewer CUs idle
+// and need fewer cuts (128- against 64-row blocks): 256 tokens over 1 000 keys 26.0 / 19.9, a
+// 500-token prompt 16.3 / 14.3, at head_dim 256 44.7 / 26.7, 1 000 tokens there 58.8 / 43.6; not
+// down to a few tiles (head_dim 256, 7 prompts of 137 tokens 20.4 / 21.0).
 constexpr int64_t kTileLongCap = 4096;
+constexpr int64_t kTileShortCap = 1024;  // twice as much at head_dim 256
 int tile_row_waves(int64_t batch, int64_t num_kv_heads, int64_t rows, int64_t head_dim,
                    int64_t cap, int64_t num_cus) {
   if (rows <= 64) return 2;
+  if (cap > 256 && cap <= (head_dim == 256 ? 2 : 1) * kTileShortCap &&
+      batch * num_kv_heads * ceil_div(rows, 128) <= num_cus / 2)
+    return 2;
   if (head_dim == 256 || rows <= 128) return 4;
   const int64_t units8 = batch * num_kv_heads * ceil_div(rows, 256);
   return units8 >= num_cus || cap >= kTileLongCap ? 8 : 4;

@@ -623,6 +623,20 @@ def test_tiled_plan_block_rows_and_pieces(B, Hq, Hkv, D, sq, cap, rows, pieces):
     assert p["launches"] == (2 if pieces > 2 else 1)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,D,sq,cap,rows", [
+    (1, 32, 8, 128, 256, 1008, 64),    # 64 blocks of 128 rows would leave most CUs idle
+    (1, 32, 8, 128, 500, 512, 64),
+    (1, 16, 2, 256, 1000, 1008, 64),
+    (1, 32, 8, 128, 1000, 1008, 128),  # 256 blocks of 128 rows
+    (7, 16, 2, 256, 137, 144, 128),    # a few tiles of keys
+])
+def test_short_keys_take_64_row_blocks(B, Hq, Hkv, D, sq, cap, rows):
+    """Fewer than half a round of 128-row blocks: 64-row ones, and one piece each."""
+    p = plan(B, Hq, Hkv, D, 16, -(-cap // 16), num_cus=256, seqlen_q=sq)
+    assert p["schedule"] == "tiled" and p["splits"] == 1, p
+    assert p["workgroups"] == B * Hkv * -(-sq * (Hq // Hkv) // rows)
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,D,sq", [(16, 128, 1, 128, 1), (64, 128, 1, 128, 1),
                                            (8, 32, 8, 128, 16), (1, 32, 8, 128, 512),
                                            (256, 128, 1, 128, 1), (16, 16, 2, 256, 4)])
