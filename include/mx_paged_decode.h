@@ -81,8 +81,9 @@ extern "C" {
                                       K/V tiles shared through LDS, long key ranges cut into
                                       pieces merged in the same launch (plans of up to two) or a
                                       second one: automatic plans of more than 32 query rows per
-                                      KV head (more than 16 at head_dim 256), where the workspace
-                                      holds its partials                                          */
+                                      KV head (more than 16 at head_dim 256; there not 256 rows
+                                      and more over short keys), where the workspace holds its
+                                      partials                                                    */
 
 /* Phase flags for mx_paged_gqa_decode (0 = run everything). */
 #define MX_PHASE_MAIN_ONLY 1        /* split grid: run only the split-KV kernel, partials stay in

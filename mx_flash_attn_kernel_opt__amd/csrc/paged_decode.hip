@@ -3111,6 +3111,20 @@ void plan_tiled(int64_t batch, int64_t seqlen_q, int64_t num_heads, int64_t num_
   set_tile_parts(parts, batch, seqlen_q * num_heads, head_dim, plan);
 }
 
+// Head dim 256, a few hundred rows of few heads over short keys: the streaming kernel's passes of 16
+// rows re-read K/V that fit an XCD's L2, and need no cut; the tiled kernel has one wave per SIMD
+// and few blocks, which have to be cut.  While the passes are at most one round of workgroups (three
+// 201-token prompts, 606 passes: 31.9 / 22.3).  Streaming against tiled (us), 2 KV heads of 8 query heads:
+// a 64-token chunk over 900 keys 14.1 / 22.0, over 2 000 (131 MB of passes) 22.0 / 25.1; a
+// 500-token prompt (262 MB) 27.8 / 26.6.
+bool stream_reads_cache(int64_t batch, int64_t num_kv_heads, int64_t head_dim, int64_t rows,
+                        int64_t cap, int64_t num_cus) {
+  const int64_t passes = ceil_div(rows, 16);
+  if (head_dim != 256 || rows < 256 || batch * num_kv_heads * passes > num_cus) return false;
+  const int64_t kv_bytes = batch * num_kv_heads * cap * head_dim * 4;
+  return kv_bytes <= (int64_t(4) << 20) && kv_bytes * passes <= int64_t(140) << 20;
+}
+
 // The plan of a call: the streaming plan, or the tiled one where the call allows it (tile_ok) and
 // has the rows for it.
 int make_plan(int64_t batch, int64_t seqlen_q, int64_t num_heads, int64_t num_kv_heads,
@@ -3122,7 +3136,8 @@ int make_plan(int64_t batch, int64_t seqlen_q, int64_t num_heads, int64_t num_kv
       seqlen_q * (num_heads / num_kv_heads) < tile_min_rows(head_dim))
     return st;
   if (num_cus <= 0) st = query_num_cus(&num_cus);
-  if (st == MX_STATUS_OK)
+  if (st == MX_STATUS_OK && !stream_reads_cache(batch, num_kv_heads, head_dim, plan->rows,
+                                                plan->cap_tokens, num_cus))
     plan_tiled(batch, seqlen_q, num_heads, num_kv_heads, head_dim, num_cus, plan);
   return st;
 }

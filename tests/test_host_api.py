@@ -637,6 +637,18 @@ def test_short_keys_take_64_row_blocks(B, Hq, Hkv, D, sq, cap, rows):
     assert p["workgroups"] == B * Hkv * -(-sq * (Hq // Hkv) // rows)
 
 
+@pytest.mark.parametrize("B,sq,cap,tiled", [
+    (1, 64, 912, False), (1, 64, 2000, False), (1, 150, 160, False),
+    (1, 500, 512, True),    # 262 MB of passes
+    (3, 201, 208, True),    # more passes than CUs
+    (1, 64, 8000, True),    # K/V beyond an XCD's L2
+    (1, 20, 912, True),     # 160 rows
+])
+def test_head_dim_256_rows_over_cached_keys_stay_on_the_streaming_kernels(B, sq, cap, tiled):
+    p = plan(B, 16, 2, 256, 16, -(-cap // 16), num_cus=256, seqlen_q=sq)
+    assert (p["schedule"] == "tiled") == tiled, p
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,D,sq", [(16, 128, 1, 128, 1), (64, 128, 1, 128, 1),
                                            (8, 32, 8, 128, 16), (1, 32, 8, 128, 512),
                                            (256, 128, 1, 128, 1), (16, 16, 2, 256, 4)])
