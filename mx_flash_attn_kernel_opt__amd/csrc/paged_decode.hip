@@ -3029,6 +3029,13 @@ constexpr double kTileCutUs = 20.;
 // blocks: one piece 23.8, two merged in the launch 26.1, four in a second one 20.9).
 double tile_fixed_us(int64_t pieces) { return pieces > kTileFusedPieces ? 4. : 8.; }
 
+// n equal pieces (fewer, where whole tiles make it so) of the capacity.
+void set_tile_pieces(int64_t n, int64_t head_dim, Plan* plan) {
+  const int64_t kb = tile_keys_of(head_dim, plan->tile_row_waves);
+  const int64_t tiles = ceil_div(plan->cap_tokens, kb);
+  plan->splits = ceil_div(tiles, ceil_div(tiles, n));
+  plan->tokens_per_split = ceil_div(tiles, plan->splits) * kb;
+}
 // A tiled plan's partials, `parts` batch pieces (no more than the batch: nothing is cut and none are
 // kept), and its workspace.
 int64_t tile_bytes(int64_t parts, int64_t batch, int64_t seq_rows, int64_t head_dim) {
@@ -3053,7 +3060,6 @@ void plan_tiled(int64_t batch, int64_t seqlen_q, int64_t num_heads, int64_t num_
   const int64_t cap = plan->cap_tokens;
   const int wr = tile_row_waves(batch, num_kv_heads, plan->rows, head_dim, cap, num_cus);
   const int64_t kb = tile_keys_of(head_dim, wr);
-  const int64_t cap_tiles = ceil_div(cap, kb);
   plan->schedule = MX_SCHEDULE_TILED;
   plan->tile_row_waves = wr;
   plan->row_tiles = ceil_div(plan->rows, 32 * wr);
@@ -3077,13 +3083,11 @@ void plan_tiled(int64_t batch, int64_t seqlen_q, int64_t num_heads, int64_t num_
       best_us = us;
     }
   }
-  const int64_t per_piece = ceil_div(cap_tiles, best);
-  int64_t ns = ceil_div(cap_tiles, per_piece);
+  set_tile_pieces(best, head_dim, plan);
   if (batch > kTileCutBatch || units * ceil_div(kTileMaxPieces, kMergeFanIn) > kMaxSlots ||
-      batch * ns * seqlen_q * num_heads * head_dim * 4 > kMaxHandoffBytes)
-    ns = 1;
-  plan->splits = ns;
-  plan->tokens_per_split = ns > 1 ? per_piece * kb : cap_tiles * kb;
+      batch * plan->splits * seqlen_q * num_heads * head_dim * 4 > kMaxHandoffBytes)
+    set_tile_pieces(1, head_dim, plan);
+  const int64_t ns = plan->splits;
   plan->groups = plan->slots = 0;
   // 64 rows or fewer, one block per head, and more units than run at once: the lengths decide which
   // workgroups end last, so the longest sequences start first (64 sequences of 1 000-4 000
@@ -3627,13 +3631,39 @@ int prepare_decode(const void* q, const void* k_cache, const void* v_cache, cons
                    max_pages_per_seq, max_seq_len, num_splits, 0, pair_ok, false, plan);
     if (st != MX_STATUS_OK) return st;
   }
-  if (*workspace != nullptr) {
-    if (workspace_bytes < plan->workspace_bytes)
-      return fail(MX_STATUS_WORKSPACE_TOO_SMALL,
-                  "workspace_bytes " + std::to_string(workspace_bytes) + " < required " +
-                      std::to_string(plan->workspace_bytes));
-    return MX_STATUS_OK;
+  const bool fits = *workspace != nullptr
+                        ? workspace_bytes >= plan->workspace_bytes
+                        : internal_workspace(plan->workspace_bytes,
+                                             static_cast<hipStream_t>(stream),
+                                             workspace) == MX_STATUS_OK;
+  if (fits) return MX_STATUS_OK;
+  if (tile_ok && num_splits == 0 && plan->rows >= tile_min_rows(head_dim)) {
+    // Less than either plan asks for: a tiled plan of as many pieces as fit, if two do.
+    int64_t cus = 0;
+    Plan tiled;
+    const int64_t seq_rows = seqlen_q * num_heads;
+    if (query_num_cus(&cus) == MX_STATUS_OK &&
+        make_stream_plan(batch, seqlen_q, num_heads, num_kv_heads, head_dim, page_size,
+                         max_pages_per_seq, max_seq_len, 0, cus, pair_ok, &tiled) ==
+            MX_STATUS_OK) {
+      plan_tiled(batch, seqlen_q, num_heads, num_kv_heads, head_dim, cus, &tiled);
+      for (int64_t n = tiled.splits; n >= 2; --n) {
+        const int64_t need = tile_bytes(n * batch, batch, seq_rows, head_dim);
+        if (*workspace != nullptr ? workspace_bytes < need
+                                  : internal_workspace(need, static_cast<hipStream_t>(stream),
+                                                       workspace) != MX_STATUS_OK)
+          continue;
+        set_tile_pieces(n, head_dim, &tiled);
+        set_tile_parts(tiled.splits * batch, batch, seq_rows, head_dim, &tiled);
+        *plan = tiled;
+        return MX_STATUS_OK;
+      }
+    }
   }
+  if (*workspace != nullptr)
+    return fail(MX_STATUS_WORKSPACE_TOO_SMALL,
+                "workspace_bytes " + std::to_string(workspace_bytes) + " < required " +
+                    std::to_string(plan->workspace_bytes));
   return internal_workspace(plan->workspace_bytes, static_cast<hipStream_t>(stream), workspace);
 }
 

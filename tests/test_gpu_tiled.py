@@ -259,6 +259,29 @@ def test_workspace_of_the_reported_size_serves_every_scale(lens, G, D, sq):
         assert_close_to_oracle(out, ref, f"scale {scale} in {p['workspace_bytes']} bytes")
 
 
+@pytest.mark.parametrize("lens,G,D,sq,pieces", [
+    ([700], 16, 128, 64, 4), ([512, 100], 128, 128, 3, 2),  # one piece less than the plan's, or two
+    ([800], 1, 256, 256, 5),       # the plan is a streaming one of 6 splits
+])
+def test_workspace_of_fewer_pieces_serves(lens, G, D, sq, pieces):
+    """Room for fewer pieces than the tiled plan's and less than the streaming plan's: the call runs
+    as many as fit; with room for less than two it is refused."""
+    inp = _inputs(lens, G, 1, D, 16, sq, seed=D)
+    s, p = inp.spec, _plan(inp)
+    part = s.batch * sq * s.num_heads * 4
+    need = (229632 + -(-pieces * part // 256) * 256) + pieces * part * D
+    assert need < p["workspace_bytes"], (need, p)
+    ref = _oracle(inp, True)
+    ws = make_workspace(need, DEV)
+    out = _run(inp, causal=True, workspace=ws)
+    assert_close_to_oracle(out, ref, f"{pieces} pieces of {p}")
+    assert torch.equal(out, _run(inp, causal=True, workspace=ws))
+    assert read_device_status(ws) == 0
+    with pytest.raises(_lib.MXAttnError) as e:
+        _run(inp, causal=True, workspace=make_workspace(229632 + part, DEV))
+    assert e.value.status == _lib.MX_STATUS_WORKSPACE_TOO_SMALL
+
+
 def test_bad_pages_and_long_lengths_are_flagged():
     inp = _inputs([300, 130], 8, 2, 128, 16, 8, seed=13, max_pages=20)
     bt, lens = inp.block_table.clone(), inp.seq_lens.clone()
