@@ -2718,7 +2718,7 @@ struct Plan {
   int tile_row_waves = 0;         // MX_SCHEDULE_TILED: row waves per workgroup (32 rows each)
   bool longest_first = false;     // MX_SCHEDULE_TILED: sequences by descending length
   bool cut = false;               // MX_SCHEDULE_TILED: pieces cut by the batch's lengths
-  int64_t tile_parts = 0;         // MX_SCHEDULE_TILED: batch pieces its partials hold (0: no partials)
+  int64_t tile_parts = 0;         // MX_SCHEDULE_TILED: batch pieces its partials hold (0: none)
   int64_t cut_slots = 0;          // (MainShape)
   double cut_tile_us = 0.;
   double cut_merge_us = 0.;
@@ -3002,8 +3002,8 @@ constexpr int64_t kTileFusedPieces = 2;
 // over 2K keys 47.5 / 46.4 / 43.9; 64 tokens over 8K keys 31.6 / 29.4 / 30.4, each at its best
 // piece count).  At head_dim 256 a wave takes a SIMD's registers: four waves, two or four on rows.
 //
-// Up to half a round of 128-row blocks over short keys takes 64-row blocks, which leave fewer CUs idle
-// and need fewer cuts (128- against 64-row blocks): 256 tokens over 1 000 keys 26.0 / 19.9, a
+// Up to half a round of 128-row blocks over short keys takes 64-row blocks, which leave fewer CUs
+// idle and need fewer cuts (128- against 64-row blocks): 256 tokens over 1 000 keys 26.0 / 19.9, a
 // 500-token prompt 16.3 / 14.3, at head_dim 256 44.7 / 26.7, 1 000 tokens there 58.8 / 43.6; not
 // down to a few tiles (head_dim 256, 7 prompts of 137 tokens 20.4 / 21.0).
 constexpr int64_t kTileLongCap = 4096;
@@ -3025,8 +3025,8 @@ int tile_row_waves(int64_t batch, int64_t num_kv_heads, int64_t rows, int64_t he
 // in a table of 128K tokens, 630 us a piece, 79 and 36; 256 sequences of log-uniform lengths up
 // to 8 160 143 and 66; 512 tokens over 2 000 keys in a table of 32K tokens 70 and 38.
 constexpr double kTileCutUs = 20.;
-// The combine launch, or the merge in the main one, in the model (256 tokens over 1 000 keys in 128-row
-// blocks: one piece 23.8, two merged in the launch 26.1, four in a second one 20.9).
+// The combine launch, or the merge in the main one, in the model (256 tokens over 1 000 keys in
+// 128-row blocks: one piece 23.8, two merged in the launch 26.1, four in a second one 20.9).
 double tile_fixed_us(int64_t pieces) { return pieces > kTileFusedPieces ? 4. : 8.; }
 
 // n equal pieces (fewer, where whole tiles make it so) of the capacity.
@@ -3036,8 +3036,8 @@ void set_tile_pieces(int64_t n, int64_t head_dim, Plan* plan) {
   plan->splits = ceil_div(tiles, ceil_div(tiles, n));
   plan->tokens_per_split = ceil_div(tiles, plan->splits) * kb;
 }
-// A tiled plan's partials, `parts` batch pieces (no more than the batch: nothing is cut and none are
-// kept), and its workspace.
+// A tiled plan's partials, `parts` batch pieces (no more than the batch: nothing is cut and none
+// are kept), and its workspace.
 int64_t tile_bytes(int64_t parts, int64_t batch, int64_t seq_rows, int64_t head_dim) {
   return parts <= batch ? kStatusBytes
                         : kPartialBase + align_up(parts * seq_rows * 4, 256) +

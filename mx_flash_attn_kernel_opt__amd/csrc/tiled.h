@@ -70,8 +70,8 @@ __device__ __forceinline__ float tile_launch_us(float count, float slots_inv, fl
   return fminf(rounds * longest, total * slots_inv + longest);
 }
 
-// How a batch is cut (MainShape::cut_rows > 0), from its lengths alone and not from the capacity, which
-// is the block table's width and often far beyond them: the longest sequence into n
+// How a batch is cut (MainShape::cut_rows > 0), from its lengths alone and not from the capacity,
+// which is the block table's width and often far beyond them: the longest sequence into n
 // pieces, every other one into pieces of at most that many tiles, for the n of 1 .. kTileMaxPieces
 // whose modelled time is shortest among those with at most cut_rows pieces in the batch and, if
 // n > 1, at least kTileMinPieceKeys keys in one.  Grid row y is the batch's y-th piece.
@@ -161,7 +161,8 @@ __device__ __forceinline__ TileCut cut_tiles_of(const int32_t* __restrict__ seq_
   const bool ok = n == 1 || (pieces <= sh.cut_rows && top * kb >= n * kTileMinPieceKeys);
   // (Positive floats order as their bits do; n in the low ones, the least of equal times.)
   const uint32_t best =
-      wave_min((as_u32(ok ? fmaxf(us, 0.f) : INFINITY) & ~(kTileMaxPieces - 1u)) + (uint32_t)(n - 1));
+      wave_min((as_u32(ok ? fmaxf(us, 0.f) : INFINITY) & ~(kTileMaxPieces - 1u)) +
+               (uint32_t)(n - 1));
   per = __builtin_amdgcn_readlane(per, best % kTileMaxPieces);
   const double inv = piece_inverse(per);
   const uint32_t mine2 = count(per, inv);
@@ -252,11 +253,12 @@ struct TileTree {
 //
 // What bounds it: with many rows per head the work is two matrix products, 4 * D flop per row and
 // key, so K and V are read once per 32*WR rows (the streaming kernels: per 16 or 32) and shared
-// through LDS.  A 4 096-token prompt (Hq=32, Hkv=8, D=128) runs at 970 TFLOP/s of bf16 MFMA,
-// where a large library product reaches 1 240-1 360 on the same card; the streaming kernels ran
-// it at 135.  Per tile of 64 keys a wave issues 32 MFMAs (1 024 cycles) and 180 other VALU
-// instructions, LDS serves 8 waves x 32 KB at up to 256 bytes per cycle, and two waves per SIMD
-// (210-230 registers at head_dim 128) cover each other's softmax and waits.
+// through LDS.  A 4 096-token prompt (Hq=32, Hkv=8, D=128) takes 154 us as a whole call without an
+// append, 892 TFLOP/s, where a large library product reaches 1 240-1 360 on the same card; the
+// streaming kernels ran it at 135.  The matrix cores are busy 37 % of the cycles.  Per tile of 64
+// keys a wave issues 32 MFMAs (1 024 cycles) and 180 other VALU instructions, LDS serves 8 waves
+// x 32 KB at up to 256 bytes per cycle, and two waves per SIMD (236-239 registers at head_dim
+// 128, no scratch) cover each other's softmax and waits.
 //
 //  * QK is S^T = K . Q^T in 32x32x16 MFMAs: the result leaves lane (row r32, half hi) the scores of
 //    keys 4*hi + {0..3, 8..11, 16..19, 24..27} of its own query row, so the row maximum is 31
@@ -272,8 +274,6 @@ struct TileTree {
 //    sequence's end are stored to LDS as zero V.  A wave skips tiles past its rows' last key.
 //  * One code path for masked and full tiles: instantiated twice, the compiler hoisted both tiles'
 //    operands and spilled (head_dim 128: 276 bytes per lane, 2.3 times slower).
-//  * Scratch: 20 bytes a lane at head_dim 256 with a fused bf16 append in 64-row blocks, outside the
-//    tile loop; none in the others.
 
 template <int D, int WR, bool kFp8, bool kAppend>
 __global__ __launch_bounds__(64 * tile_waves<D>())

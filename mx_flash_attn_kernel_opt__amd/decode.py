@@ -275,7 +275,8 @@ class BoundDecode:
     ``__call__(phase=0)`` issues the launch(es) on the bound stream and raises on a bad
     status.  The bound tensors must stay alive and keep their storage.  ``plan`` is the shape's
     plan (``plan()``); a call that plan does not serve (a score scale below 1e-30, or a workspace
-    too small for a tiled plan's partials) runs a streaming schedule instead.
+    too small for a tiled plan's partials) runs a streaming schedule or a plan of fewer pieces
+    instead.
     """
 
     def __init__(self, q, k_cache, v_cache, block_table, seq_lens, scale=None, *, out=None,
