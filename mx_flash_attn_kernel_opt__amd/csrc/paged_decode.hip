@@ -1575,12 +1575,7 @@ __device__ __forceinline__ void merge_group(const Tree& tree, int gslot, int str
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));
   const int total = nrows * (D / 4);
-  // (Trees with blocks of many rows: as many elements as keep 32 loads of four floats in flight.)
-  constexpr int E = Tree::kElems * W <= 32 ? Tree::kElems : 32 / W;
-  if (E > 2 && total > 2 * 64 * NW) {
-    for (int e0 = tid; e0 < total; e0 += (E > 2 ? E : 2) * 64 * NW)
-      merge_elems<D, NW, W, (E > 2 ? E : 2)>(tree, e0, total, gslot, stride, gsize, final, s_lse);
-  } else if (total > 64 * NW && W <= 16) {
+  if (total > 64 * NW && W <= 16) {
     for (int e0 = tid; e0 < total; e0 += 2 * 64 * NW)
       merge_elems<D, NW, W, 2>(tree, e0, total, gslot, stride, gsize, final, s_lse);
   } else {
@@ -1649,7 +1644,6 @@ __device__ __forceinline__ void merge_tree(const Tree& tree, int item, int nitem
 // the counter region holds split_groups = ceil(num_splits / kMergeFanIn) counters per unit.
 template <int D>
 struct SplitTree {
-  static constexpr int kElems = 2;
   const MainShape& sh;
   float* part_o;
   float* part_lse;
@@ -1870,7 +1864,6 @@ void mx_paged_decode_splitkv(
 // enough for 8^4 = 4096 pieces per unit), indexed like the slots.  A slot holds tile_rows rows.
 template <int D>
 struct BalancedTree {
-  static constexpr int kElems = 2;
   const MainShape& sh;
   float* part_o;
   float* part_lse;

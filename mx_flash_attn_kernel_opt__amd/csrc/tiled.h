@@ -214,13 +214,9 @@ __device__ __forceinline__ TileSlots tile_slots(int first, int b, const MainShap
   return TileSlots{1, (int64_t)(first - b) * seq_rows, seq_rows};
 }
 
-// The merge tree over the pieces of a row block (merge_tree).  A block has up to 256 rows for its
-// threads and few pieces: a thread merges up to kElems elements per round trip (two pieces of
-// 128-row blocks, 256 tokens over 1 000 keys: 28.4 -> 26.0 us a call against 2 elements).
+// The merge tree over the pieces of a row block (merge_tree).
 template <int D>
 struct TileTree {
-  // (head_dim 64 has 128 registers at most; at 256 the merge's would cost the main loop.)
-  static constexpr int kElems = D == 128 ? 8 : 2;
   const MainShape& sh;
   float* part_o;
   float* part_lse;
@@ -257,7 +253,7 @@ struct TileTree {
 // append, 892 TFLOP/s, where a large library product reaches 1 240-1 360 on the same card; the
 // streaming kernels ran it at 135.  The matrix cores are busy 37 % of the cycles.  Per tile of 64
 // keys a wave issues 32 MFMAs (1 024 cycles) and 180 other VALU instructions, LDS serves 8 waves
-// x 32 KB at up to 256 bytes per cycle, and two waves per SIMD (236-239 registers at head_dim
+// x 32 KB at up to 256 bytes per cycle, and two waves per SIMD (200-230 registers at head_dim
 // 128, no scratch) cover each other's softmax and waits.
 //
 //  * QK is S^T = K . Q^T in 32x32x16 MFMAs: the result leaves lane (row r32, half hi) the scores of
